@@ -815,7 +815,7 @@ def mid_bench(P, hip, n_boards=4096, seed=2, tune=True, plain=True):
         # plain time / this floor unless the kernels read less than the algorithmic bytes
         "roofline": {"bound": "hbm", "achieved": work / batched_s / 1e9, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                      "frac": work / batched_s / 1e9 / HBM_PEAK_GBPS, "traffic": mid_traffic(),
-                     "kernel": "batched plan (mid_level1_kernel, mid_boards_kernel, mid_prep_kernel)",
+                     "kernel": "batched plan (mid_step_kernel, mid_boards_kernel, mid_prep_kernel)",
                      "bytes_per_run": work, "run_ms": batched_s * 1e3},
         "hbm_floor_s": floor_s,
         "max_batched_over_plain_at_hbm_peak": plain_s / floor_s if plain_s else None,

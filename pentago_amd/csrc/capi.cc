@@ -51,19 +51,18 @@ pe_status device_tables(DevTables* out, std::string* err) {
   std::lock_guard<std::mutex> lock(g_dev_mutex);
   if (g_dev_ready[dev]) { *out = g_dev[dev]; return PE_OK; }
   const Tables* T;
+  const MidTabsHost* M;
   try {
     T = &tables();
+    M = &mid_tabs();
   } catch (const std::exception& e) {
     *err = e.what();
     return PE_ERR_TABLES;
   }
-  // unpacked rotation-minimal quadrants and choose(n, k)
+  // unpacked rotation-minimal quadrants
   std::vector<uint32_t> sides(T->rmin_flat_size);
   for (int i = 0; i < T->rmin_flat_size; i++)
     sides[i] = uint32_t(T->unpack[T->rmin_flat[i]][0]) | uint32_t(T->unpack[T->rmin_flat[i]][1]) << 16;
-  std::vector<int32_t> choose(32 * 32);
-  for (int n = 0; n < 32; n++)
-    for (int k = 0; k < 32; k++) choose[n * 32 + k] = choose_host(n, k);
   // log2 of the number of local rotations fixing a quadrant: 2 if a quarter turn fixes both
   // sides, 1 if only a half turn does, else 0 (pentago/base/count.cc:235-245)
   std::vector<uint8_t> stab(T->rmin_flat_size);
@@ -77,11 +76,14 @@ pe_status device_tables(DevTables* out, std::string* err) {
   build_field_pool(&pool);
   const size_t sizes[] = {sizeof T->superwin, sizeof(uint16_t) * size_t(T->rmin_flat_size),
                           sizeof(uint32_t) * sides.size(), sizeof T->rmin_inverse, sizeof T->pack,
-                          sizeof T->commute, sizeof(int32_t) * choose.size(), stab.size(),
-                          sizeof(uint64_t) * pool.size()};
-  const void* srcs[] = {T->superwin, T->rmin_flat, sides.data(), T->rmin_inverse, T->pack, T->commute, choose.data(),
-                        stab.data(), pool.data()};
-  constexpr int kParts = 9;
+                          sizeof T->commute, stab.size(), sizeof(uint64_t) * pool.size(),
+                          sizeof(MidSched) * M->sched.size(), sizeof(MidTile) * M->tiles.size(),
+                          sizeof(uint32_t) * M->bases.size(),
+                          sizeof(MidClass) * M->classes.size(), sizeof(Kids) * M->kids.size()};
+  const void* srcs[] = {T->superwin, T->rmin_flat, sides.data(), T->rmin_inverse, T->pack, T->commute,
+                        stab.data(), pool.data(), M->sched.data(), M->tiles.data(), M->bases.data(),
+                        M->classes.data(), M->kids.data()};
+  constexpr int kParts = 13;
   size_t total = 0, offs[kParts];
   for (int i = 0; i < kParts; i++) { offs[i] = total; total += (sizes[i] + 255) & ~size_t(255); }
   void* d = nullptr;
@@ -100,9 +102,13 @@ pe_status device_tables(DevTables* out, std::string* err) {
   D.rmin_inverse = reinterpret_cast<const uint16_t*>(b + offs[3]);
   D.pack = reinterpret_cast<const uint16_t*>(b + offs[4]);
   D.commute = reinterpret_cast<const uint8_t*>(b + offs[5]);
-  D.choose = reinterpret_cast<const int32_t*>(b + offs[6]);
-  D.rmin_stab = b + offs[7];
-  D.fields = reinterpret_cast<const uint64_t*>(b + offs[8]);
+  D.rmin_stab = b + offs[6];
+  D.fields = reinterpret_cast<const uint64_t*>(b + offs[7]);
+  D.mid.sched = reinterpret_cast<const MidSched*>(b + offs[8]);
+  D.mid.tiles = reinterpret_cast<const MidTile*>(b + offs[9]);
+  D.mid.bases = reinterpret_cast<const uint32_t*>(b + offs[10]);
+  D.mid.classes = reinterpret_cast<const MidClass*>(b + offs[11]);
+  D.mid.kids = reinterpret_cast<const Kids*>(b + offs[12]);
   g_dev[dev] = D;
   g_dev_ready[dev] = true;
   *out = D;

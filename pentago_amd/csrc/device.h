@@ -8,6 +8,7 @@
 #include <string>
 
 #include "../../include/pentago_amd.h"
+#include "mid_tiles.h"
 
 namespace pe {
 
@@ -19,9 +20,9 @@ struct DevTables {
   const uint16_t* rmin_inverse; // 19683 entries
   const uint16_t* pack;         // 512 entries
   const uint8_t* commute;       // 8*256 entries
-  const int32_t* choose;        // choose(n, k) at [n*32 + k], n,k < 32
   const uint8_t* rmin_stab;     // per rotation-minimal quadrant: log2 of its local stabilizer size
   const uint64_t* fields;       // field pool of the fused end kernels (end.h: field_pool_off)
+  MidTabs mid;                  // tiles of the midsolve
 };
 
 // Upload the tables to the current device (idempotent per device).

@@ -1,5 +1,5 @@
-// Midsolve host side: per-board constants and result traversal (own implementation of
-// pentago/mid/internal.h:37-69 and pentago/mid/midengine.cc:127-158).
+// Midsolve host side: board validation and result traversal (own implementation of
+// pentago/mid/internal.h:37-47 and pentago/mid/midengine.cc:127-158).
 #include "mid.h"
 
 #include <algorithm>
@@ -44,33 +44,7 @@ bool make_mid_info(const pe_high_board& b, MidInfo* I) {
   if (I->spots > 18) return false;
   const uint64_t empty = mask & ~(b.side[0] | b.side[1]);
   for (int i = 0, k = 0; i < 64; i++) if (empty >> i & 1) I->empty[k++] = uint8_t(i);
-  const int ws = bottleneck(I->spots);
-  I->workspace = ws;
-  for (int n = 0; n <= I->spots; n++) {
-    const int k0 = n >> 1, k1 = n - k0;
-    const int sets0 = choose_host(I->spots, k0), sets1 = choose_host(I->spots, k1);
-    const int sets0p = choose_host(I->spots - k1, k0), sets1p = choose_host(I->spots - k0, k1);
-    I->sets0_off[n + 1] = I->sets0_off[n] + sets0;
-    I->sets1p_off[n + 1] = I->sets1p_off[n] + sets1p;
-    I->cs1ps_off[n + 1] = I->cs1ps_off[n] + sets1p * (I->spots - k0);
-    I->wins1_off[n + 1] = I->wins1_off[n] + sets1;
-    I->spaces[n].ny = sets0p;
-    I->spaces[n].size = sets1 * sets0p;
-    I->spaces[n].lo = (n & 1) ? ws - sets1 * sets0p : 0;
-    I->positions[n] = int64_t(sets0) * sets1p;
-  }
-  I->spaces[I->spots + 1] = MidGrab{0, 0, 0};
   return true;
-}
-
-MidSizes mid_sizes(const MidInfo& I) {
-  MidSizes s;
-  s.set0 = I.sets0_off[I.spots + 1];
-  s.wins1 = I.wins1_off[I.spots + 1];
-  s.cs1ps = I.cs1ps_off[I.spots + 1];
-  s.set1p = I.sets1p_off[I.spots + 1];
-  s.work = I.workspace;
-  return s;
 }
 
 // ---- high board (pentago/high/board.cc) ----

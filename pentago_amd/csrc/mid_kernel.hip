@@ -1,11 +1,8 @@
 // Midsolve kernels for gfx950.
 //
-// Per board: one table-building pass (per-s0 tables, the other side's wins, child index
-// remaps; pentago/mid/internal.h:122-259) and then one sweep per level n = spots..0 in
-// which one thread evaluates one position (s0, s1p) exactly as internal.h:358-408 does,
-// carrying (win, notlose) together.  Consecutive threads share s0 and walk s1p, so the
-// children they OR (rows child_s0s[i] of the previous level) are read as nearly contiguous
-// runs.
+// Per board: one pass building the wins tables (pentago/mid/internal.h:122-131) and then one
+// launch per step of tiles (mid_tiles.h), a workgroup per tile, carrying (win, notlose)
+// together.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -31,106 +28,58 @@ __device__ __forceinline__ int find_board(const int64_t* prefix, int nb, int64_t
   return lo;
 }
 
-// The binomial table (4 KB) is staged in LDS first: the subset unranking and the offset
-// loops below read it in chains of dependent lookups.
 __global__ __launch_bounds__(256) void mid_prep_kernel(const MidBoardDev* __restrict__ boards,
                                                        const int64_t* __restrict__ prefix, int nb,
                                                        int64_t total, DevTables T) {
-  __shared__ int32_t sC[32 * 32];
-  for (int i = threadIdx.x; i < 32 * 32; i += blockDim.x) sC[i] = T.choose[i];
-  __syncthreads();
   const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t >= total) return;
   const int b = find_board(prefix, nb, t);
-  mid_prep_entry(boards[b], t - prefix[b], T, sC);
+  mid_wins_entry(boards[b], t - prefix[b], T);
 }
 
-// Level launches of one board are spread over the 8 XCDs (workgroup i runs on XCD i % 8) by
-// bands of s1p: XCD x sweeps every s0 for bands x, x + 8, ... in turn.  A position's
-// children sit in the rows of the next level at columns that follow its s1p, so an XCD's L2
-// then holds its band of each row instead of every XCD touching every column.
-__device__ __forceinline__ bool banded_position(uint32_t wg, uint32_t tid, uint32_t band, uint32_t nsets1p,
-                                                uint32_t nsets0, int64_t* pos) {
-  const int64_t q = int64_t(wg >> 3) * 256 + tid;
-  const int64_t per_band = int64_t(nsets0) * band;
-  const int64_t bi = q / per_band;
-  const int64_t r = q - bi * per_band;
-  const int64_t s0 = r / band;
-  const int64_t s1p = (int64_t(wg & 7) + 8 * bi) * band + (r - s0 * band);
-  if (s1p >= nsets1p) return false;   // a band past the last, or the last band's tail
-  *pos = s0 * nsets1p + s1p;
-  return true;
-}
-
-// step: level n = spots_b - step for every board with spots_b >= step
-// band > 0 (one board only): banded order, see banded_position
-__global__ __launch_bounds__(256) void mid_level_kernel(const MidBoardDev* __restrict__ boards,
-                                                        const int64_t* __restrict__ prefix, int nb,
-                                                        int64_t total, int step, LevelGrid g, DevTables T) {
-  if (g.band) {
-    int64_t pos;
-    if (!banded_position(blockIdx.x, threadIdx.x, g.band, g.nsets1p, g.nsets0, &pos)) return;
-    mid_position(boards[0], boards[0].I.spots - step, pos, boards[0].work, T);
-    return;
-  }
-  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= total) return;
-  const int b = find_board(prefix, nb, t);
+// Step `step` of every board that has one: workgroup w sweeps tile w - prefix[b] of the
+// step's tiles of board b.
+// Workgroup i runs on XCD i % 8: each XCD takes runs of neighbouring tiles, which read the same
+// tiles.  Runs of 1 / 4 / 16 / 64 tiles measured within 3 %, 16 the fastest; one run of an eighth
+// of the launch to each XCD is 20 % slower (the groups of a step differ in tile size).
+constexpr int kRun = 16;
+// A step that writes more than this (24 KB a tile at most) than the L2s hold together, 32 MB, is
+// stored past them: 18 empty cells 2.51 -> 2.43 ms; a small step's reader finds it in the L2.
+constexpr int kStreamTiles = 2048;
+__global__ __launch_bounds__(kTileThreads, 5) void mid_step_kernel(const MidBoardDev* __restrict__ boards,
+                                                                const int64_t* __restrict__ prefix, int nb,
+                                                                int step, int ntiles, MidTabs M) {
+  __shared__ TileLds lds;
+  const int x = blockIdx.x & 7, y = blockIdx.x >> 3;
+  const int w = (y / kRun * 8 + x) * kRun + y % kRun;
+  if (w >= ntiles) return;
+  const int b = nb == 1 ? 0 : find_board(prefix, nb, w);
+  const int t = w - (nb == 1 ? 0 : int(prefix[b]));
   const MidBoardDev& B = boards[b];
-  mid_position(B, B.I.spots - step, t - prefix[b], B.work, T);
-}
-
-__global__ __launch_bounds__(256) void mid_level1_kernel(const MidBoardDev* __restrict__ board, int n,
-                                                         int64_t positions, LevelGrid g, DevTables T) {
-  int64_t t;
-  if (g.band) {
-    if (!banded_position(blockIdx.x, threadIdx.x, g.band, g.nsets1p, g.nsets0, &t)) return;
-  } else {
-    t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= positions) return;
-  }
-  mid_position(*board, n, t, board->work, T);
+  const MidSched& S = M.sched[B.I.spots];
+  mid_tile(tile_job(B, B.work, S, M, ntiles > kStreamTiles), M, S.first[step] + t, lds, int(threadIdx.x));
 }
 
 }  // namespace
 
-LevelGrid level_grid(const MidInfo& I, int n) {
-  const int64_t positions = I.positions[n];
-  const uint32_t n1 = uint32_t(I.sets1p_off[n + 1] - I.sets1p_off[n]);
-  LevelGrid g;
-  g.blocks = unsigned((positions + 255) / 256);
-  g.band = 0;
-  g.nsets1p = n1;
-  g.nsets0 = n1 ? uint32_t(positions / n1) : 0;
-  const uint32_t band = std::min<uint32_t>(kLevelBand, (n1 + 7) / 8);
-  if (kLevelBand == 0 || band < 16 || positions < (int64_t(1) << 16)) return g;   // small levels: linear order
-  const uint32_t nbands = (n1 + band - 1) / band;
-  const int64_t per_xcd = int64_t((nbands + 7) / 8) * g.nsets0 * band;
-  g.band = band;
-  g.blocks = unsigned(8 * ((per_xcd + 255) / 256));
-  return g;
+int mid_steps(const MidInfo& I) { return mid_tabs().sched[size_t(I.spots)].steps; }
+int64_t mid_step_tiles(const MidInfo& I, int step) {
+  const MidSched& S = mid_tabs().sched[size_t(I.spots)];
+  return step < S.steps ? S.first[step + 1] - S.first[step] : 0;
 }
 
 // Allocation of one board's device scratch inside a caller-provided arena.
 static size_t align256(size_t x) { return (x + 255) & ~size_t(255); }
 
-size_t mid_table_bytes(const MidInfo& I) {
-  const MidSizes s = mid_sizes(I);
-  return align256(sizeof(Set0Info) * s.set0) + align256(sizeof(Wins1) * s.wins1) +
-         align256(sizeof(uint16_t) * s.cs1ps) + align256(sizeof(uint32_t) * s.set1p);
-}
-size_t mid_work_bytes(const MidInfo& I) { return align256(32 * size_t(mid_sizes(I).work)); }
+size_t mid_table_bytes(const MidInfo& I) { return size_t(mid_table_area_bytes(I.spots)); }
+size_t mid_work_bytes(const MidInfo& I) { return align256(32 * size_t(mid_work_entries(I.spots))); }
 size_t mid_board_bytes(const MidInfo& I) {
   return mid_table_bytes(I) + mid_work_bytes(I) + align256(sizeof(pe_halfsupers) * 19);
 }
 
 void mid_carve_tables(MidBoardDev* B, uint8_t* base) {
-  const MidSizes s = mid_sizes(B->I);
-  size_t off = 0;
-  B->set0 = reinterpret_cast<Set0Info*>(base + off); off += align256(sizeof(Set0Info) * s.set0);
-  B->wins1 = reinterpret_cast<Wins1*>(base + off); off += align256(sizeof(Wins1) * s.wins1);
-  B->cs1ps = reinterpret_cast<uint16_t*>(base + off); off += align256(sizeof(uint16_t) * s.cs1ps);
-  B->set1p_bits = reinterpret_cast<uint32_t*>(base + off);
+  B->wins = reinterpret_cast<uint64_t*>(base);
+  B->spill = B->wins + (size_t(8) << B->I.spots);   // 2 << spots entries of 4 words
 }
 
 void mid_carve(MidBoardDev* B, uint8_t* base) {
@@ -140,12 +89,13 @@ void mid_carve(MidBoardDev* B, uint8_t* base) {
   B->results = reinterpret_cast<pe_halfsupers*>(base + t + mid_work_bytes(B->I));
 }
 
-pe_status mid_launch_level(const MidBoardDev* board, const MidInfo& info, int n, int64_t positions,
-                           const DevTables& T, hipStream_t stream) {
-  if (positions <= 0) return PE_OK;
-  const LevelGrid g = level_grid(info, n);
-  hipLaunchKernelGGL(mid_level1_kernel, dim3(g.blocks), dim3(256), 0, stream, board, n, positions, g, T);
-  PE_HIP(hipGetLastError(), "mid_level1_kernel launch");
+pe_status mid_launch_step(const MidBoardDev* board, const MidInfo& info, int step, const DevTables& T,
+                          hipStream_t stream) {
+  const int64_t tiles = mid_step_tiles(info, step);
+  if (tiles <= 0) return PE_OK;
+  hipLaunchKernelGGL(mid_step_kernel, dim3(unsigned((tiles + 8 * kRun - 1) / (8 * kRun) * (8 * kRun))), dim3(kTileThreads), 0, stream, board, nullptr, 1, step,
+                     int(tiles), T.mid);
+  PE_HIP(hipGetLastError(), "mid_step_kernel launch");
   return PE_OK;
 }
 
@@ -171,27 +121,20 @@ pe_status mid_solve_levels(const std::vector<MidInfo>& infos, uint8_t* arena, st
   std::vector<MidBoardDev> boards(nb);
   result_offsets->resize(nb);
   size_t off = 0;
-  int max_spots = 0;
+  int steps = 0;
   for (int b = 0; b < nb; b++) {
     boards[b].I = infos[b];
     mid_carve(&boards[b], arena + off);
     (*result_offsets)[b] = size_t(reinterpret_cast<uint8_t*>(boards[b].results) - arena);
     off += mid_board_bytes(infos[b]);
-    max_spots = std::max(max_spots, infos[b].spots);
+    steps = std::max(steps, mid_steps(infos[b]));
   }
-  // prefix sums: prep entries, then positions per step
-  const int steps = max_spots + 1;
+  // prefix sums: prep entries, then tiles per step
   std::vector<int64_t> prefix(size_t(nb + 1) * (steps + 1), 0);
-  for (int b = 0; b < nb; b++) {
-    const MidSizes s = mid_sizes(infos[b]);
-    prefix[b + 1] = prefix[b] + s.set0 + s.wins1 + s.set1p;
-  }
+  for (int b = 0; b < nb; b++) prefix[b + 1] = prefix[b] + mid_prep_entries(infos[b]);
   for (int t = 0; t < steps; t++) {
     int64_t* p = prefix.data() + size_t(nb + 1) * (t + 1);
-    for (int b = 0; b < nb; b++) {
-      const int n = infos[b].spots - t;
-      p[b + 1] = p[b] + (n >= 0 ? infos[b].positions[n] : 0);
-    }
+    for (int b = 0; b < nb; b++) p[b + 1] = p[b] + mid_step_tiles(infos[b], t);
   }
   const size_t desc_bytes = sizeof(MidBoardDev) * nb;
   const size_t bytes = desc_bytes + sizeof(int64_t) * prefix.size();
@@ -219,13 +162,10 @@ pe_status mid_solve_levels(const std::vector<MidInfo>& infos, uint8_t* arena, st
     const int64_t* p = prefix.data() + size_t(nb + 1) * (t + 1);
     const int64_t total = p[nb];
     if (total <= 0) continue;
-    LevelGrid g;
-    g.blocks = unsigned((total + 255) / 256);
-    g.band = g.nsets1p = g.nsets0 = 0;
-    if (nb == 1) g = level_grid(infos[0], infos[0].spots - t);
-    hipLaunchKernelGGL(mid_level_kernel, dim3(g.blocks), dim3(256), 0, stream, dboards,
-                       dprefix + size_t(nb + 1) * (t + 1), nb, total, t, g, T);
-    PE_HIP(hipGetLastError(), "mid_level_kernel launch");
+    if (total > 0x7fff0000) { set_error("too many tiles in one midsolve launch"); return PE_ERR_CAPACITY; }
+    hipLaunchKernelGGL(mid_step_kernel, dim3(unsigned((total + 8 * kRun - 1) / (8 * kRun) * (8 * kRun))), dim3(kTileThreads), 0, stream, dboards,
+                       dprefix + size_t(nb + 1) * (t + 1), nb, t, int(total), T.mid);
+    PE_HIP(hipGetLastError(), "mid_step_kernel launch");
   }
   if (!desc_cache) PE_HIP(hipFreeAsync(d, stream), "hipFreeAsync(mid descriptors)");
   return PE_OK;
@@ -247,11 +187,11 @@ constexpr int kScratchDevices = 64;
 std::mutex g_scratch_mu[kScratchDevices];      // one solve at a time per device in this process
 uint8_t* g_scratch_ptr[kScratchDevices];       // device address of `scratch` on each device
 
-// The descriptors of one board's launches: the board record, then the prefix sums the prep
-// and level kernels read (mid_solve_levels' layout for one board: [0, entries] per launch).
+// The descriptors of one board's launches: the board record, then the prefix the prep kernel
+// reads ([0, entries]).
 struct NoAllocDesc {
   MidBoardDev board;
-  int64_t prefix[2 * 21];
+  int64_t prefix[2];
 };
 
 }  // namespace
@@ -285,15 +225,12 @@ pe_status mid_solve_noalloc(const pe_high_board& hb, pe_halfsupers* results, hip
   }
   uint8_t* const base = g_scratch_ptr[dev];
   // every table, workspace and result entry the kernels read is written by them first
-  // (prep, then level n = spots .. 0), so nothing in the array needs clearing between calls
+  // (prep, then the tile layers), so nothing in the array needs clearing between calls
   NoAllocDesc d;
   std::memset(&d, 0, sizeof d);
   d.board.I = I;
   mid_carve(&d.board, base + desc_bytes);
-  const MidSizes sz = mid_sizes(I);
-  const int steps = I.spots + 1;
-  d.prefix[1] = sz.set0 + sz.wins1 + sz.set1p;
-  for (int t = 0; t < steps; t++) d.prefix[2 * (t + 1) + 1] = I.positions[I.spots - t];
+  d.prefix[1] = mid_prep_entries(I);
   // every way out waits for the work queued on the stream: the descriptors are read from
   // this frame, and the next call (on any stream) reuses the array
   struct Drain {
@@ -303,19 +240,9 @@ pe_status mid_solve_noalloc(const pe_high_board& hb, pe_halfsupers* results, hip
   PE_HIP(hipMemcpyAsync(base, &d, sizeof d, hipMemcpyHostToDevice, stream), "hipMemcpyAsync(descriptors)");
   const auto* dboard = reinterpret_cast<const MidBoardDev*>(base);
   const auto* dprefix = reinterpret_cast<const int64_t*>(base + offsetof(NoAllocDesc, prefix));
-  if (d.prefix[1] > 0) {
-    hipLaunchKernelGGL(mid_prep_kernel, dim3(unsigned((d.prefix[1] + 255) / 256)), dim3(256), 0, stream, dboard,
-                       dprefix, 1, d.prefix[1], T);
-    PE_HIP(hipGetLastError(), "mid_prep_kernel launch");
-  }
-  for (int t = 0; t < steps; t++) {
-    const int64_t total = d.prefix[2 * (t + 1) + 1];
-    if (total <= 0) continue;
-    const LevelGrid g = level_grid(I, I.spots - t);
-    hipLaunchKernelGGL(mid_level_kernel, dim3(g.blocks), dim3(256), 0, stream, dboard, dprefix + 2 * (t + 1), 1, total,
-                       t, g, T);
-    PE_HIP(hipGetLastError(), "mid_level_kernel launch");
-  }
+  pe_status st = mid_launch_prep(dboard, dprefix, 1, d.prefix[1], T, stream);
+  for (int k = 0; k < mid_steps(I) && st == PE_OK; k++) st = mid_launch_step(dboard, I, k, T, stream);
+  if (st != PE_OK) return st;
   PE_HIP(hipMemcpyAsync(results, d.board.results, sizeof(pe_halfsupers) * 19, hipMemcpyDeviceToHost, stream),
          "hipMemcpyAsync(results)");
   PE_HIP(hipStreamSynchronize(stream), "allocation-free midsolve");

@@ -2,10 +2,10 @@
 //
 // A batch is split by size.  Small boards (at most small_spots empty cells) are solved whole
 // by one workgroup each: a persistent kernel whose workgroups pop board indices from a device
-// queue (one atomic counter) and sweep every level of the board with workgroup barriers
-// between levels, in a workspace slot owned by the workgroup.  No workgroup ever waits for
-// another.  Large boards run level by level on one or more streams of their own (table pass,
-// then one launch per level over the whole device), boards of one stream reusing that
+// queue (one atomic counter) and sweep every tile of the board (mid_tiles.h) with workgroup
+// barriers between its steps, in a workspace slot owned by the workgroup.  No workgroup ever
+// waits for another.  Large boards run step by step on one or more streams of their own (wins
+// tables, then one launch per step over the whole device), boards of one stream reusing that
 // stream's slot in stream order.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -65,7 +65,7 @@ struct MidPlan {
   std::vector<hipStream_t> streams;    // owned, layout.streams of them
   std::vector<hipEvent_t> events;      // fork + one join per stream
   hipGraphExec_t graph_exec = nullptr;
-  int64_t launches = 0;                // kernel launches per run
+  int64_t launches = 0;                // kernel launches per run, at most
 };
 
 // alloc_stream null: synchronous hipMalloc/hipMemcpy; else stream-ordered on it.  With
@@ -99,26 +99,19 @@ void mid_server_destroy(MidServer* S);
 size_t mid_table_bytes(const MidInfo& I);
 size_t mid_work_bytes(const MidInfo& I);
 size_t mid_board_bytes(const MidInfo& I);
-// Lay out one board's tables (mid_table_bytes) at `base`; or tables, workspace and results
+// Lay out one board's table area (mid_table_bytes) at `base`; or tables, workspace and results
 // (mid_board_bytes) at `base`.
 void mid_carve_tables(MidBoardDev* B, uint8_t* base);
 void mid_carve(MidBoardDev* B, uint8_t* base);
 // One launch building the tables of every board: prefix[b] = prep entries before board b.
 pe_status mid_launch_prep(const MidBoardDev* boards, const int64_t* prefix, int nb, int64_t total,
                           const DevTables& T, hipStream_t stream);
-// Launch shape of one level of one board: `band` > 0 spreads the level over the XCDs by bands
-// of s1p columns (blocks counts the padded grid), 0 keeps the linear order.  Measured on
-// 2048 boards of 18..30 stones, batched: linear 1.14 s; bands of 4 / 8 / 12 / 16 / 24 / 32
-// columns 1.22 / 0.99 / 0.96 / 0.95 / 0.98 / 0.99 s, one band per XCD 1.01 s; bands 16 wide
-// dealt to the XCDs in contiguous runs instead of in turn 1.05 s.
-constexpr uint32_t kLevelBand = 16;
-struct LevelGrid {
-  unsigned blocks;
-  uint32_t band, nsets1p, nsets0;
-};
-LevelGrid level_grid(const MidInfo& I, int n);
-// One launch sweeping level n of one board (all positions).
-pe_status mid_launch_level(const MidBoardDev* board, const MidInfo& info, int n, int64_t positions,
-                           const DevTables& T, hipStream_t stream);
+// Threads of a prep launch for one board; steps of a board; tiles of one step (0 past the last).
+inline int64_t mid_prep_entries(const MidInfo& I) { return int64_t(2) << I.spots; }
+int mid_steps(const MidInfo& I);
+int64_t mid_step_tiles(const MidInfo& I, int step);
+// One launch sweeping the tiles of one step of one board.
+pe_status mid_launch_step(const MidBoardDev* board, const MidInfo& info, int step, const DevTables& T,
+                          hipStream_t stream);
 
 }  // namespace pe

@@ -1,5 +1,5 @@
 // Batched midsolve: small boards through a persistent one-workgroup-per-board kernel fed
-// by a device queue, large boards level by level on their own streams (see mid_queue.h).
+// by a device queue, large boards step by step on their own streams (see mid_queue.h).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -16,14 +16,18 @@ namespace {
 
 __global__ void mid_head_reset_kernel(unsigned int* head) { *head = 0; }
 
-// Workgroups pop small boards from `head` and sweep all their levels; workgroup w owns the
-// workspace slot work_base + w * work_stride.  Levels are separated by workgroup barriers,
-// which order the global-memory writes of one level before the reads of the next.
+// Workgroups pop small boards from `head` and sweep all their tiles, one at a time
+// for each kTileThreads threads; workgroup w owns the workspace slot work_base + w * work_stride.  Steps are separated
+// by full workgroup barriers, which order the global-memory writes of one step before the reads
+// of the next.
 template <int kThreads>
-__global__ __launch_bounds__(kThreads) void mid_boards_kernel(const MidBoardDev* __restrict__ boards, int nboards,
-                                                              uint8_t* __restrict__ work_base, int64_t work_stride,
-                                                              unsigned int* __restrict__ head, DevTables T) {
+__global__ __launch_bounds__(kThreads, 4) void mid_boards_kernel(const MidBoardDev* __restrict__ boards, int nboards,
+                                                                 uint8_t* __restrict__ work_base, int64_t work_stride,
+                                                                 unsigned int* __restrict__ head, MidTabs M) {
+  constexpr int kSub = kThreads / kTileThreads;
+  __shared__ TileLds lds[kSub];
   __shared__ int s_b;
+  const int sub = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kTileThreads);
   uint64_t* work = reinterpret_cast<uint64_t*>(work_base + int64_t(blockIdx.x) * work_stride);
   for (;;) {
     if (threadIdx.x == 0) s_b = int(atomicAdd(head, 1u));
@@ -32,10 +36,13 @@ __global__ __launch_bounds__(kThreads) void mid_boards_kernel(const MidBoardDev*
     __syncthreads();
     if (b >= nboards) return;
     const MidBoardDev& B = boards[b];
-    const int spots = B.I.spots;
-    for (int n = spots; n >= 0; n--) {
-      const int positions = int(B.I.positions[n]);
-      for (int p = threadIdx.x; p < positions; p += kThreads) mid_position(B, n, p, work, T);
+    const MidSched& S = M.sched[B.I.spots];
+    const TileJob J = tile_job(B, work, S, M, false);
+    for (int k = 0; k < S.steps; k++) {
+      for (int t = S.first[k]; t < S.first[k + 1]; t += kSub) {
+        mid_tile(J, M, t + sub < S.first[k + 1] ? t + sub : -1, lds[sub], int(threadIdx.x) % kTileThreads);
+        tile_barrier();   // before the next tile's wins replace this one's
+      }
       __syncthreads();
     }
   }
@@ -59,7 +66,9 @@ const char* mid_layout(const std::vector<MidInfo>& infos, const MidConfig& cfg, 
   const int nb = int(infos.size());
   if (cfg.threads != 256 && cfg.threads != 512 && cfg.threads != 1024) return "threads must be 256, 512 or 1024";
   for (int b = 0; b < nb; b++) (infos[b].spots <= cfg.small_spots ? L->small : L->big).push_back(b);
-  std::stable_sort(L->big.begin(), L->big.end(), [&](int a, int b) { return infos[a].spots > infos[b].spots; });
+  // largest first: a workgroup's last board is then a small one
+  for (std::vector<int>* v : {&L->small, &L->big})
+    std::stable_sort(v->begin(), v->end(), [&](int a, int b) { return infos[a].spots > infos[b].spots; });
   // descriptor blob
   L->o_big = up256(sizeof(MidBoardDev) * L->small.size());
   L->o_prefix = L->o_big + up256(sizeof(MidBoardDev) * L->big.size());
@@ -148,8 +157,7 @@ pe_status mid_plan_create(const std::vector<MidInfo>& infos, const MidConfig& cf
     B.work = nullptr;   // the workgroup's slot
     B.results = res + 19 * size_t(L.small[k]);
     std::memcpy(&sdev[k], &B, sizeof B);
-    const MidSizes s = mid_sizes(B.I);
-    prefix[k + 1] = prefix[k] + s.set0 + s.wins1 + s.set1p;
+    prefix[k + 1] = prefix[k] + mid_prep_entries(B.I);
   }
   plan->small_prep_total = prefix[L.small.size()];
   plan->big_prep_total.resize(L.big.size());
@@ -162,10 +170,9 @@ pe_status mid_plan_create(const std::vector<MidInfo>& infos, const MidConfig& cf
     B.work = reinterpret_cast<uint64_t*>(slot + mid_table_bytes(B.I));
     B.results = res + 19 * size_t(L.big[k]);
     std::memcpy(&bdev[k], &B, sizeof B);
-    const MidSizes s = mid_sizes(B.I);
     int64_t* p = prefix + L.small.size() + 1 + 2 * k;
     p[0] = 0;
-    p[1] = s.set0 + s.wins1 + s.set1p;
+    p[1] = mid_prep_entries(B.I);
     plan->big_prep_total[k] = p[1];
   }
   if (alloc_stream && upload && blob.size() <= upload_bytes) {
@@ -218,15 +225,15 @@ pe_status launch_small(const MidPlan& plan, hipStream_t s) {
   switch (plan.cfg.threads) {
     case 256:
       hipLaunchKernelGGL(mid_boards_kernel<256>, grid, dim3(256), 0, s, plan.small_dev, n, work, stride, plan.head,
-                         plan.tables);
+                         plan.tables.mid);
       break;
     case 512:
       hipLaunchKernelGGL(mid_boards_kernel<512>, grid, dim3(512), 0, s, plan.small_dev, n, work, stride, plan.head,
-                         plan.tables);
+                         plan.tables.mid);
       break;
     default:
       hipLaunchKernelGGL(mid_boards_kernel<1024>, grid, dim3(1024), 0, s, plan.small_dev, n, work, stride, plan.head,
-                         plan.tables);
+                         plan.tables.mid);
   }
   PE_HIP(hipGetLastError(), "mid_boards_kernel launch");
   return PE_OK;
@@ -238,8 +245,8 @@ pe_status launch_big(const MidPlan& plan, size_t k, hipStream_t s) {
   const MidBoardDev* B = plan.big_dev + k;
   pe_status st = mid_launch_prep(B, plan.prefix + L.small.size() + 1 + 2 * k, 1, plan.big_prep_total[k], plan.tables, s);
   if (st != PE_OK) return st;
-  for (int n = I.spots; n >= 0; n--) {
-    st = mid_launch_level(B, I, n, I.positions[n], plan.tables, s);
+  for (int n = 0; n < mid_steps(I); n++) {
+    st = mid_launch_step(B, I, n, plan.tables, s);
     if (st != PE_OK) return st;
   }
   return PE_OK;

@@ -348,24 +348,25 @@ PE_HD H2 split_half(S4 s, int parity) {
   }
   return h;
 }
-PE_HD H2 halfsuper_wins(uint64_t side, int parity, const uint64_t* table) {
-  return split_half(super_wins<true>(side, table), parity);
-}
-// rmax on halves; flips parity (pentago/mid/halfsuper.h:18-42, 155-203).
-PE_HD uint64_t hrmax_lo(uint64_t x) {
-  const uint64_t t = (x | (x >> 1)) & 0x5555555555555555ull;
-  const uint64_t y0 = t | (t << 1);                               // parity quadrant
-  const uint64_t y1 = ((x << 2) & 0xFCFCFCFCFCFCFCFCull) | ((x << 6) & 0xC0C0C0C0C0C0C0C0ull) |
-                      ((x >> 2) & 0x3F3F3F3F3F3F3F3Full) | ((x >> 6) & 0x0303030303030303ull);
-  const uint64_t y2 = ((x << 8) & 0xFFFFFF00FFFFFF00ull) | ((x << 24) & 0xFF000000FF000000ull) |
-                      ((x >> 8) & 0x00FFFFFF00FFFFFFull) | ((x >> 24) & 0x000000FF000000FFull);
-  return y0 | y1 | y2;
+// rmax on halves; flips parity (pentago/mid/halfsuper.h:18-42, 155-203).  One 32-bit word per
+// r3: the other parity of a pair of r0, the neighbours in r1 (two-bit groups of a byte), r2
+// (bytes) and r3 (words); ORed with `extra`.
+PE_HD uint32_t rot32(uint32_t x, int k) { return x >> k | x << (32 - k); }
+PE_HD uint32_t hrmax_word(uint32_t x, uint32_t below, uint32_t above, uint32_t extra) {
+  const uint32_t pair = lop3_32<kSel>(x >> 1, x << 1, 0x55555555u);          // x itself is ORed in below
+  const uint32_t w = x | lop3_32<kSel>(x >> 4, x << 4, 0x0F0F0F0Fu);         // r1 and r1 + 2
+  const uint32_t side = lop3_32<kSel>(w >> 2, w << 2, 0x33333333u);          // both neighbours of r1
+  return lop3_32<kOr3>(lop3_32<kOr3>(lop3_32<kOr3>(x, pair, side), below, above),
+                       lop3_32<kOr3>(rot32(x, 8), rot32(x, 24), extra), 0u);
 }
 PE_HD H2 hrmax(H2 h) {
-  const uint64_t a = h.w[0], b = h.w[1];
-  const uint64_t y3 = (a << 32) | (a >> 32) | (b << 32) | (b >> 32);
-  H2 r; r.w[0] = hrmax_lo(a) | y3; r.w[1] = hrmax_lo(b) | y3;
-  return r;
+  const uint32_t x[4] = {uint32_t(h.w[0]), uint32_t(h.w[0] >> 32), uint32_t(h.w[1]), uint32_t(h.w[1] >> 32)};
+  uint32_t r[4];
+  for (int d = 0; d < 4; d++) r[d] = hrmax_word(x[d], x[(d + 3) & 3], x[(d + 1) & 3], 0);
+  H2 o;
+  o.w[0] = r[0] | uint64_t(r[1]) << 32;
+  o.w[1] = r[2] | uint64_t(r[3]) << 32;
+  return o;
 }
 
 }  // namespace pe
