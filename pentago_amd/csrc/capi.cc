@@ -45,6 +45,58 @@ std::atomic<int> g_end_form[kMaxDevices];
 
 void set_error(const std::string& e) { g_error = e; }
 
+namespace {
+struct Kept { void* ptr = nullptr; size_t cap = 0; };
+std::mutex g_kept_mu;
+Kept g_kept[kMaxDevices];
+
+// The kept block of the current device, if it passes `fits`; the caller owns it then.
+template <class F>
+Kept kept_out(F fits) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return Kept();
+  std::lock_guard<std::mutex> lock(g_kept_mu);
+  const Kept k = g_kept[dev];
+  if (!k.ptr || !fits(k)) return Kept();
+  g_kept[dev] = Kept();
+  return k;
+}
+}  // namespace
+
+hipError_t device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) return e;
+  const Kept k = kept_out([](const Kept&) { return true; });
+  if (!k.ptr) return e;
+  (void)hipGetLastError();
+  (void)hipFree(k.ptr);
+  return hipMalloc(p, bytes);
+}
+
+hipError_t block_take(size_t bytes, size_t limit, void** p, size_t* cap) {
+  const Kept k = kept_out([&](const Kept& b) { return b.cap >= bytes && b.cap <= limit && b.cap / 2 < bytes; });
+  if (k.ptr) {
+    *p = k.ptr;
+    *cap = k.cap;
+    return hipSuccess;
+  }
+  *cap = std::min(std::max(limit, bytes), bytes + bytes / 8);
+  const hipError_t e = device_malloc(p, *cap);
+  if (e == hipSuccess || *cap == bytes) return e;
+  (void)hipGetLastError();
+  *cap = bytes;
+  return device_malloc(p, bytes);
+}
+
+void block_give(int device, void* p, size_t cap) {
+  if (cap <= kKeptBytes && device >= 0 && device < kMaxDevices) {   // the newer block stays
+    std::lock_guard<std::mutex> lock(g_kept_mu);
+    std::swap(g_kept[device].ptr, p);
+    g_kept[device].cap = cap;
+  }
+  if (p) (void)hipFree(p);
+}
+
 pe_status device_tables(DevTables* out, std::string* err) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) { *err = "no HIP device"; return PE_ERR_DEVICE; }
@@ -87,7 +139,7 @@ pe_status device_tables(DevTables* out, std::string* err) {
   size_t total = 0, offs[kParts];
   for (int i = 0; i < kParts; i++) { offs[i] = total; total += (sizes[i] + 255) & ~size_t(255); }
   void* d = nullptr;
-  if (hipMalloc(&d, total) != hipSuccess) { *err = "hipMalloc(tables) failed"; return PE_ERR_DEVICE; }
+  if (device_malloc(&d, total) != hipSuccess) { *err = "hipMalloc(tables) failed"; return PE_ERR_DEVICE; }
   for (int i = 0; i < kParts; i++)
     if (hipMemcpy(static_cast<uint8_t*>(d) + offs[i], srcs[i], sizes[i], hipMemcpyHostToDevice) != hipSuccess) {
       (void)hipFree(d);
@@ -535,9 +587,9 @@ pe_status pe_end_compute_line_host(const pe_line* line, const void* h_input, voi
     void*& a; void*& b;
     ~Free() { if (a) (void)hipFree(a); if (b) (void)hipFree(b); }
   } free_bufs{din, dout};
-  PE_HIP(hipMalloc(&dout, out_bytes), "hipMalloc(output)");
+  PE_HIP(device_malloc(&dout, out_bytes), "hipMalloc(output)");
   if (in_bytes) {
-    PE_HIP(hipMalloc(&din, in_bytes), "hipMalloc(input)");
+    PE_HIP(device_malloc(&din, in_bytes), "hipMalloc(input)");
     PE_HIP(hipMemcpy(din, h_input, in_bytes, hipMemcpyHostToDevice), "hipMemcpy(input)");
   }
   PE_HIP(hipMemset(dout, 0, out_bytes), "hipMemset(output)");

@@ -32,6 +32,19 @@ bool device_tables_ready(DevTables* out);
 
 void set_error(const std::string& e);
 
+// hipMalloc that gives the kept block (below) back to the device before it fails.
+hipError_t device_malloc(void** p, size_t bytes);
+
+// Memory of a finished plan, kept for the next one: at most one block a device, of at most
+// kKeptBytes.  Freed VRAM is cleared before it is handed out again, which costs a process that
+// makes a plan a batch about 27 ms a GB once the device has no clean memory left.
+// take: a block for `bytes` (its size in *cap, at most `limit` and less than twice `bytes`), the
+// kept one of the current device or a new one with an eighth to spare.  give: back from its
+// owner, who has waited for all work that uses it.  Thread-safe: a block has one owner.
+constexpr size_t kKeptBytes = size_t(4) << 30;
+hipError_t block_take(size_t bytes, size_t limit, void** p, size_t* cap);
+void block_give(int device, void* p, size_t cap);
+
 // Grow-only device allocation reused across synchronous calls (callers serialize use and
 // have no work pending on it when it grows).
 struct DeviceBuffer {
@@ -42,7 +55,7 @@ struct DeviceBuffer {
     if (ptr) (void)hipFree(ptr);
     ptr = nullptr;
     cap = 0;
-    const hipError_t e = hipMalloc(&ptr, bytes);
+    const hipError_t e = device_malloc(&ptr, bytes);
     if (e == hipSuccess) cap = bytes;
     return e;
   }

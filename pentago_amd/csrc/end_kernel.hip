@@ -221,7 +221,7 @@ pe_status plan_create(const std::vector<LineHost>& lines, EndPlan* plan) {
   const size_t off_refl = off_offs + sizeof(int64_t) * offs.size();
   const size_t bytes = off_refl + refl.size();
   void* d = nullptr;
-  PE_HIP(hipMalloc(&d, bytes), "hipMalloc(line plan)");
+  PE_HIP(device_malloc(&d, bytes), "hipMalloc(line plan)");
   auto* base = static_cast<uint8_t*>(d);
   const int64_t* doffs = reinterpret_cast<const int64_t*>(base + off_offs);
   for (int k = 0; k < n; k++) {

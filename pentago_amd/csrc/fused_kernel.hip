@@ -516,7 +516,7 @@ static pe_status pack_fused_plan(const std::vector<BlockDev>& blocks, const std:
   const size_t o_heads = o_refl + up(refl.size());
   const size_t bytes = o_heads + 256;
   void* d = nullptr;
-  if (hipMalloc(&d, bytes) != hipSuccess) { *err = "hipMalloc(fused plan) failed"; return PE_ERR_DEVICE; }
+  if (device_malloc(&d, bytes) != hipSuccess) { *err = "hipMalloc(fused plan) failed"; return PE_ERR_DEVICE; }
   auto* base = static_cast<uint8_t*>(d);
   for (size_t k = 0; k < devs.size(); k++) devs[k].in_off = reinterpret_cast<const int64_t*>(base + o_offs) + at[k];
   std::vector<uint8_t> blob(bytes, 0);
@@ -937,7 +937,7 @@ pe_status line_tabs(const LineHost& h, LineTabs* out, std::string* err) {
     if (need > C.left) {
       const size_t chunk = std::max<size_t>(need, size_t(4) << 20);
       void* p = nullptr;
-      if (hipMalloc(&p, chunk) != hipSuccess) { *err = "hipMalloc(line move tables) failed"; return PE_ERR_DEVICE; }
+      if (device_malloc(&p, chunk) != hipSuccess) { *err = "hipMalloc(line move tables) failed"; return PE_ERR_DEVICE; }
       C.chunk = static_cast<uint8_t*>(p);
       C.left = chunk;
     }

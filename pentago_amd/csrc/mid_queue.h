@@ -53,6 +53,9 @@ struct MidPlan {
   std::vector<MidInfo> infos;
   hipStream_t alloc_stream = nullptr;  // stream-ordered allocation (serving) or null
   uint8_t* mem = nullptr;              // layout.bytes
+  size_t mem_cap = 0;                  // block_take's size when the plan holds such a block, else 0
+  hipEvent_t done = nullptr;           // the end of the last run, for such a block
+  bool captured = false;               // a run was captured: nobody knows when the memory is free
   bool owns_mem = true;                // false: caller memory, not freed by the plan
   const MidBoardDev* small_dev = nullptr;
   const MidBoardDev* big_dev = nullptr;
@@ -82,7 +85,8 @@ pe_status mid_plan_run(MidPlan& plan, hipStream_t stream);
 // synchronized, mid_plan_zero_tail clears the entries past each board's spots.
 pe_status mid_plan_copy_results(const MidPlan& plan, pe_halfsupers (*out)[19], hipStream_t stream);
 void mid_plan_zero_tail(const MidPlan& plan, pe_halfsupers (*out)[19]);
-// Frees the plan's memory (stream-ordered on alloc_stream when it was allocated that way).
+// Gives the plan's memory back (stream-ordered on alloc_stream when it was allocated that way,
+// else block_give).
 void mid_plan_destroy(MidPlan* plan);
 int mid_board_blocks_per_cu(int threads);
 

@@ -139,7 +139,7 @@ pe_status mid_plan_create(const std::vector<MidInfo>& infos, const MidConfig& cf
   plan->owns_mem = !(memory && L.bytes <= memory_bytes);
   if (!plan->owns_mem) mem = memory;
   else if (alloc_stream) PE_HIP(hipMallocAsync(&mem, L.bytes, alloc_stream), "hipMallocAsync(mid batch)");
-  else PE_HIP(hipMalloc(&mem, L.bytes), "hipMalloc(mid batch)");
+  else PE_HIP(block_take(L.bytes, size_t(cfg.budget), &mem, &plan->mem_cap), "hipMalloc(mid batch)");
   plan->mem = static_cast<uint8_t*>(mem);
   uint8_t* base = plan->mem;
   // descriptors
@@ -187,6 +187,7 @@ pe_status mid_plan_create(const std::vector<MidInfo>& infos, const MidConfig& cf
   } else {
     PE_HIP(hipMemcpy(base, blob.data(), blob.size(), hipMemcpyHostToDevice), "hipMemcpy(mid batch)");
   }
+  if (plan->mem_cap) PE_HIP(hipEventCreateWithFlags(&plan->done, hipEventDisableTiming), "hipEventCreate(mid batch)");
   plan->small_dev = reinterpret_cast<const MidBoardDev*>(base);
   plan->big_dev = reinterpret_cast<const MidBoardDev*>(base + L.o_big);
   plan->prefix = reinterpret_cast<const int64_t*>(base + L.o_prefix);
@@ -278,7 +279,9 @@ pe_status launch_all(const MidPlan& plan, hipStream_t stream) {
 
 }  // namespace
 
-pe_status mid_plan_run(MidPlan& plan, hipStream_t stream) {
+namespace {
+
+pe_status run_plan(MidPlan& plan, hipStream_t stream) {
   if (!plan.cfg.graph) return launch_all(plan, stream);
   if (!plan.graph_exec) {
     hipStream_t cap = nullptr;
@@ -303,6 +306,20 @@ pe_status mid_plan_run(MidPlan& plan, hipStream_t stream) {
   return PE_OK;
 }
 
+}  // namespace
+
+pe_status mid_plan_run(MidPlan& plan, hipStream_t stream) {
+  const pe_status st = run_plan(plan, stream);
+  if (!plan.done || plan.captured) return st;
+  hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone ||
+      hipEventRecord(plan.done, stream) != hipSuccess) {
+    (void)hipGetLastError();
+    plan.captured = true;
+  }
+  return st;
+}
+
 pe_status mid_plan_copy_results(const MidPlan& plan, pe_halfsupers (*out)[19], hipStream_t stream) {
   if (plan.nb)
     PE_HIP(hipMemcpyAsync(out, plan.results, sizeof(pe_halfsupers) * 19 * size_t(plan.nb), hipMemcpyDeviceToHost,
@@ -324,8 +341,11 @@ void mid_plan_destroy(MidPlan* plan) {
   for (hipEvent_t e : plan->events) (void)hipEventDestroy(e);
   if (plan->mem && plan->owns_mem) {
     if (plan->alloc_stream) (void)hipFreeAsync(plan->mem, plan->alloc_stream);
-    else (void)hipFree(plan->mem);
+    else if (!plan->done || plan->captured || hipEventSynchronize(plan->done) != hipSuccess) (void)hipFree(plan->mem);
+    else block_give(plan->device, plan->mem, plan->mem_cap);
   }
+  if (plan->done) (void)hipEventDestroy(plan->done);
+  plan->done = nullptr;
   plan->graph_exec = nullptr;
   plan->streams.clear();
   plan->events.clear();

@@ -200,7 +200,7 @@ struct MidServer {
       if (arena[size_t(k)]) (void)hipFree(arena[size_t(k)]);
       arena[size_t(k)] = nullptr;
       arena_cap[size_t(k)] = 0;
-      PE_HIP(hipMalloc(&arena[size_t(k)], cap), "hipMalloc(server arena)");
+      PE_HIP(device_malloc(&arena[size_t(k)], cap), "hipMalloc(server arena)");
       arena_cap[size_t(k)] = cap;
       footprint_peak = std::max(footprint_peak, int64_t(held_all_except(-1)));
     }

@@ -92,7 +92,7 @@ pe_status count_slabs(int n, const pe_slab* slabs, uint64_t (*counts)[4]) {
   if (!first[n]) return PE_OK;
   const size_t count_bytes = sizeof(uint64_t) * 4 * size_t(first[n]);
   void* d = nullptr;
-  if (hipMalloc(&d, count_bytes + count_desc_bytes(n)) != hipSuccess)
+  if (device_malloc(&d, count_bytes + count_desc_bytes(n)) != hipSuccess)
     return failed(PE_ERR_DEVICE, "hipMalloc(counts) failed");
   std::vector<uint64_t*> dst(n);
   for (int k = 0; k < n; k++) dst[k] = static_cast<uint64_t*>(d) + 4 * first[k];
@@ -288,7 +288,7 @@ pe_status pe_slice_create_in(int n, const pe_section* sections, void* arena, int
       d = static_cast<uint8_t*>(arena) + used;
       used += bytes;
     } else {
-      if (hipMalloc(&d, size_t(bytes)) != hipSuccess) {
+      if (device_malloc(&d, size_t(bytes)) != hipSuccess) {
         pe_slice_destroy(st);
         return failed(PE_ERR_CAPACITY, "hipMalloc of section " + std::to_string(k) + " failed");
       }
@@ -572,7 +572,7 @@ pe_status pe_slice_grouped_counts(int n, const pe_section* sections, int64_t bud
   const int64_t bytes = pe_slice_arena_bytes(n, sections, budget, !children);
   if (bytes < 0) return failed(PE_ERR_INVALID, "invalid sections or budget");
   void* arena = nullptr;
-  if (hipMalloc(&arena, size_t(std::max<int64_t>(bytes, 1))) != hipSuccess)
+  if (device_malloc(&arena, size_t(std::max<int64_t>(bytes, 1))) != hipSuccess)
     return failed(PE_ERR_CAPACITY, "hipMalloc(group arena) failed");
   const pe_status st = pe_slice_grouped_counts_in(n, sections, budget, children, grandchildren, counts, visit, ctx,
                                                   ngroups, arena, bytes, stream);
