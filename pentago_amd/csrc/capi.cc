@@ -126,16 +126,16 @@ pe_status device_tables(DevTables* out, std::string* err) {
   // field pool of the fused kernels (see end.h)
   std::vector<uint64_t> pool;
   build_field_pool(&pool);
+  const std::vector<uint32_t> records = mid_records(M->view());
+  const std::vector<KidRanks> kids = mid_kid_ranks(M->view());
   const size_t sizes[] = {sizeof T->superwin, sizeof(uint16_t) * size_t(T->rmin_flat_size),
                           sizeof(uint32_t) * sides.size(), sizeof T->rmin_inverse, sizeof T->pack,
                           sizeof T->commute, stab.size(), sizeof(uint64_t) * pool.size(),
-                          sizeof(MidSched) * M->sched.size(), sizeof(MidTile) * M->tiles.size(),
-                          sizeof(uint32_t) * M->bases.size(),
-                          sizeof(MidClass) * M->classes.size(), sizeof(Kids) * M->kids.size()};
+                          sizeof(MidSched) * M->sched.size(), sizeof(uint32_t) * records.size(),
+                          sizeof(KidRanks) * kids.size()};
   const void* srcs[] = {T->superwin, T->rmin_flat, sides.data(), T->rmin_inverse, T->pack, T->commute,
-                        stab.data(), pool.data(), M->sched.data(), M->tiles.data(), M->bases.data(),
-                        M->classes.data(), M->kids.data()};
-  constexpr int kParts = 13;
+                        stab.data(), pool.data(), M->sched.data(), records.data(), kids.data()};
+  constexpr int kParts = 11;
   size_t total = 0, offs[kParts];
   for (int i = 0; i < kParts; i++) { offs[i] = total; total += (sizes[i] + 255) & ~size_t(255); }
   void* d = nullptr;
@@ -157,10 +157,8 @@ pe_status device_tables(DevTables* out, std::string* err) {
   D.rmin_stab = b + offs[6];
   D.fields = reinterpret_cast<const uint64_t*>(b + offs[7]);
   D.mid.sched = reinterpret_cast<const MidSched*>(b + offs[8]);
-  D.mid.tiles = reinterpret_cast<const MidTile*>(b + offs[9]);
-  D.mid.bases = reinterpret_cast<const uint32_t*>(b + offs[10]);
-  D.mid.classes = reinterpret_cast<const MidClass*>(b + offs[11]);
-  D.mid.kids = reinterpret_cast<const Kids*>(b + offs[12]);
+  D.mid.records = reinterpret_cast<const uint32_t*>(b + offs[9]);
+  D.mid.kids = reinterpret_cast<const KidRanks*>(b + offs[10]);
   g_dev[dev] = D;
   g_dev_ready[dev] = true;
   *out = D;

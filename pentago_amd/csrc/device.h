@@ -22,7 +22,7 @@ struct DevTables {
   const uint8_t* commute;       // 8*256 entries
   const uint8_t* rmin_stab;     // per rotation-minimal quadrant: log2 of its local stabilizer size
   const uint64_t* fields;       // field pool of the fused end kernels (end.h: field_pool_off)
-  MidTabs mid;                  // tiles of the midsolve
+  MidTabsDev mid;               // tiles of the midsolve
 };
 
 // Upload the tables to the current device (idempotent per device).

@@ -6,18 +6,11 @@
 
 #include "device.h"
 #include "mid.h"
+#include "mid_queue.h"
 #include "mid_tiles.h"
 #include "super.h"
 
 namespace pe {
-
-struct MidBoardDev {
-  MidInfo I;
-  uint64_t* wins;           // [mover of the root, other][mask of empty cells]: halves of parity 0, 1
-  uint64_t* spill;          // tile entries that the workspace has no room for
-  uint64_t* work;           // tile entries, 4 u64 each
-  pe_halfsupers* results;   // 19 entries
-};
 
 // One entry of a board's wins tables: idx = player << spots | mask of empty cells, player 0 the
 // one to move at the root.  Masks with more stones than the player ever places are not read.
@@ -35,15 +28,18 @@ __device__ inline void mid_wins_entry(const MidBoardDev& B, int64_t idx, const D
   o[1] = make_ulonglong2(odd.w[0], odd.w[1]);
 }
 
-constexpr int kTileThreads = 256;   // threads that sweep one tile: the largest class at once
+constexpr int kTileThreads = 256;   // threads of a sweep, or of each of its two chains: the largest class at once
 static_assert(kTileClass <= kTileThreads, "a class is one round");
-// Loads of the tiles above in flight for a thread: slots of this tile times tiles.  2 x 4 and
-// 1 x 4 (44 registers) take 6 % and 14 % longer, 6 x 1 9 %, 6 x 2 spills.
-constexpr int kSlots = 3, kAbove = 2;
 
-// LDS of a tile: its entries as they are stored (classes of even l, then of odd l; a class's win
-// halves, then its notlose halves), and the wins of both players' stones on the low cells beside
-// the tile's high ones, halves of parity 0 and 1.
+// A level's win halves come from the notlose halves of the level below it and the other way
+// round, so a tile's entries are two chains that never meet: chain 0 is the win halves of even
+// levels and the notlose halves of odd ones (as stored, which is the other side's view, the
+// halves that those are made from), chain 1 the rest.  They are kept apart, each thread reads and
+// writes the slots of its own chain only.
+//
+// LDS of a tile: its entries as they are stored (classes of even l, then of odd l, of each chain 0,
+// then chain 1), and the wins of both players' stones on the low cells beside the tile's high
+// ones, halves of parity 0 and 1.
 struct TileLds {
   uint4 half[2 * kTileEntries];
   uint4 wins[2][2][1 << kTileCells];
@@ -57,17 +53,12 @@ __device__ __forceinline__ void tile_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-struct Two { uint4 win, nl; };   // an entry
 __device__ __forceinline__ void or4(uint4& a, const uint4& b) {
   a.x |= b.x; a.y |= b.y; a.z |= b.z; a.w |= b.w;
 }
 __device__ __forceinline__ void or4(uint4& a, const uint4& b, const uint4& c) {
   a.x = lop3_32<kOr3>(a.x, b.x, c.x); a.y = lop3_32<kOr3>(a.y, b.y, c.y);
   a.z = lop3_32<kOr3>(a.z, b.z, c.z); a.w = lop3_32<kOr3>(a.w, b.w, c.w);
-}
-__device__ __forceinline__ void or_two(Two& a, const Two& b) { or4(a.win, b.win); or4(a.nl, b.nl); }
-__device__ __forceinline__ void or_two(Two& a, const Two& b, const Two& c) {
-  or4(a.win, b.win, c.win); or4(a.nl, b.nl, c.nl);
 }
 // hrmax of four words (super.h), then OR with `extra`
 __device__ __forceinline__ uint4 hrmax4(const uint4& v, const uint4& extra) {
@@ -92,20 +83,20 @@ struct TileJob {
   uint64_t* work;
   uint64_t* spill;
   pe_halfsupers* results;
-  const MidTile* tiles;     // the board's tiles in order
-  const uint2* bases;       // first entries of a tile's halves (even levels, odd levels), by code
+  const uint32_t* records;  // of the board's tiles in order
+  const KidRanks* kids;     // rows of its number of low cells, from d = 0, l = 0 on
   int32_t ply, low, high, in_work;
   bool stream;              // entries are read again only once they have left the L2 (store_stream)
 };
-__device__ __forceinline__ TileJob tile_job(const MidBoardDev& B, uint64_t* work, const MidSched& S, const MidTabs& M,
-                                                bool stream) {
+__host__ __device__ __forceinline__ TileJob tile_job(const MidBoardDev& B, uint64_t* work, const MidSched& S,
+                                                     const MidTabsDev& M, bool stream) {
   TileJob J;
   J.wins = reinterpret_cast<const uint4*>(B.wins);
   J.work = work;
   J.spill = B.spill;
   J.results = B.results;
-  J.tiles = M.tiles + S.tiles;
-  J.bases = reinterpret_cast<const uint2*>(M.bases) + S.bases;
+  J.records = M.records + int64_t(kRecWords) * S.tiles;
+  J.kids = M.kids + mid_kid_row(S.low, 0, 0);
   J.ply = int(B.I.ply);
   J.low = S.low;
   J.high = S.high;
@@ -115,72 +106,68 @@ __device__ __forceinline__ TileJob tile_job(const MidBoardDev& B, uint64_t* work
 }
 
 // Sweep one tile (`tile` counts from the board's first; negative: only take part in the
-// barriers) with the kTileThreads threads tid = 0.. of a workgroup.  Every tile of a board runs
-// the same number of barriers (low + 2).
+// barriers) with the kTileThreads * kChains threads tid = 0.. of a workgroup: each thread both
+// chains, or with kChains = 2 the second kTileThreads threads the second chain.  Every tile of a
+// board runs the same number of barriers (low + 1).
 //
-// What bounds it: the reads of the tiles one high stone up, 32 bytes a position and empty high
-// cell.  The half that a class reads of such a tile has the same layout as the half of this tile
-// that the class is in, so all of them are ORed into the LDS first, entry by entry, with every
-// load of the tile independent of every other; the sweep that follows, a barrier a class, touches
-// the LDS only, but for the child ranks, which are loaded a class ahead.
-__device__ __forceinline__ void mid_tile(const TileJob& J, const MidTabs& M, int tile, TileLds& lds, int tid) {
-  const int wave0 = __builtin_amdgcn_readfirstlane(tid & ~63);
+// What bounds it: for a launch that fills the chip, the reads of the tiles one high stone up, 32
+// bytes a position and empty high cell; else the latency of one tile.  The half that a class
+// reads of such a tile has the same layout as the half of this tile that the class is in, so all
+// of them are ORed into the LDS first, entry by entry, with every load of the tile independent of
+// every other; the sweep that follows, a barrier a class, touches the LDS only.  The loads of a
+// tile are two deep: its record, then the children's ranks of all its classes (two registers
+// each), the wins and the tiles above at once.  Ranks loaded a class ahead and first entries
+// looked up cell by cell took 9.5 against 7.5 us for a step of 26 stones; 26 stones 68 -> 58 us,
+// 18 stones 2.57 -> 2.48 ms, 65 boards of 18-30 stones 22.5 -> 19.0 ms in all.
+template <int kChains>
+__device__ __forceinline__ void mid_tile(const TileJob& J, int tile, TileLds& lds, int tid) {
+  // Loads of the tiles above in flight for a thread: slots of this tile times tiles (a chain's
+  // slots are two rounds of its threads, both chains' three).  Both chains 2 x 4 and 1 x 4 take
+  // 6 % and 14 % longer, 6 x 1 9 %.  One chain a thread serves launches that leave the chip idle:
+  // more tiles at once.
+  constexpr int kSlots = kChains == 2 ? 2 : 3, kAbove = kChains == 2 ? 5 : 2;
+  const int chain0 = kChains == 2 ? __builtin_amdgcn_readfirstlane(tid / kTileThreads) : 0;
+  const int t = kChains == 2 ? tid % kTileThreads : tid;   // member of a class
+  const int wave0 = __builtin_amdgcn_readfirstlane(t & ~63);
   const int lane = tid & 63;
   const int low = J.low, high = J.high, spots = low + high;
-  const MidTile cfg = J.tiles[max(tile, 0)];
-  const uint32_t p = cfg.p, q = cfg.q;
+  uint32_t rec = 0;
+  if (tile >= 0 && lane < kRecWords) rec = J.records[int64_t(kRecWords) * tile + lane];
+  auto word = [&](int i) { return uint32_t(__builtin_amdgcn_readlane(int(rec), i)); };
+  const uint32_t p = word(0) & 0xffff, q = word(0) >> 16;
   const int a = __popc(p), h = a + __popc(q), d = 2 * a - h;
   const int nhigh = tile < 0 ? 0 : high - h;
+  const uint64_t counts = uint64_t(word(kRecCounts)) | uint64_t(word(kRecCounts + 1)) << 32;
+  auto count = [&](int l) { return int(counts >> (8 * l) & 0xff); };
   auto entry = [&](uint32_t e) {
-    return e < uint32_t(J.in_work) ? J.work + 4 * uint64_t(e) : J.spill + 4 * uint64_t(e - uint32_t(J.in_work));
+    return reinterpret_cast<uint4*>(e < uint32_t(J.in_work) ? J.work + 4 * uint64_t(e)
+                                                            : J.spill + 4 * uint64_t(e - uint32_t(J.in_work)));
   };
-  // lane l: class l; lane j: the tiles above with the j-th empty high cell filled by M0 (of which
-  // the odd levels are read) and by M1 (the even ones)
-  MidClass mine = {{0, 0}};
-  if (tile >= 0 && lane <= low) mine = M.classes[mid_class_row(low, d, lane)];
-  uint64_t up0 = 0, up1 = 0;
-  if (lane < nhigh) {
-    uint32_t rest = ((1u << high) - 1) & ~(p | q);
-    for (int j = 0; j < lane; j++) rest &= rest - 1;
-    uint32_t c3 = 1;
-    for (int i = __builtin_ctz(rest); i > 0; i--) c3 *= 3;
-    up0 = reinterpret_cast<uint64_t>(entry(J.bases[cfg.code + c3].y));
-    up1 = reinterpret_cast<uint64_t>(entry(J.bases[cfg.code + 2 * c3].x));
-  }
-  const uint2 own = J.bases[cfg.code];
+  KidRanks kids[kTileCells + 1];
+  const KidRanks* row = J.kids + mid_kid_row(0, d, 0) - mid_kid_row(0, 0, 0) + min(t, kTileClass - 1);
+#pragma unroll
+  for (int l = kTileCells; l >= 0; l--)
+    if (wave0 < count(l)) kids[l] = row[l * kTileClass];
   if (tile >= 0)
-    for (int i = tid; i < 4 << low; i += kTileThreads) {   // player, mask, parity
+    for (int i = tid; i < 4 << low; i += kTileThreads * kChains) {   // player, mask, parity
       const int player = i >> (low + 1), k = i & ((2 << low) - 1);
-      const uint64_t row = player ? (uint64_t(1) << spots) + (uint64_t(q) << low) : uint64_t(p) << low;
-      lds.wins[player][k & 1][k >> 1] = J.wins[2 * row + k];
+      const uint64_t first = player ? (uint64_t(1) << spots) + (uint64_t(q) << low) : uint64_t(p) << low;
+      lds.wins[player][k & 1][k >> 1] = J.wins[2 * first + k];
     }
-  auto get_class = [&](int l) {
-    MidClass c = {{0, 0}};
-    if (l >= 0)
-      for (int i = 0; i < 2; i++) c.w[i] = uint32_t(__builtin_amdgcn_readlane(int(mine.w[i]), l));
-    return c;
-  };
   // entries of the classes of even l, which come first, and of odd l
-  int size[2];
-  for (int e = 0; e < 2; e++) {
-    const MidClass top = get_class(low - ((low + e) & 1));
-    size[e] = top.at() + top.count();
-  }
+  const int size[2] = {int(word(kRecSizes) & 0xffff), int(word(kRecSizes) >> 16)};
   if (nhigh)
     for (int e = 0; e < 2; e++) {
-      const uint64_t up = (h + e) & 1 ? up1 : up0;
-      auto above = [&](int j) {
-        return reinterpret_cast<const uint4*>(uint64_t(uint32_t(__builtin_amdgcn_readlane(int(up), j))) |
-                                              uint64_t(uint32_t(__builtin_amdgcn_readlane(int(up >> 32), j))) << 32);
-      };
-      // whole waves (a lane of `up` is read only with every lane active): lanes past the end
+      const int up = kRecUp + ((h + e) & 1 ? kRecUp1 : 0);
+      const int first = chain0 * size[e], end = kChains == 2 ? first + size[e] : 2 * size[e];
+      // whole waves (a word of the record is taken with every lane active): lanes past the end
       // take the last slot once more
-      for (int i = wave0; i < 2 * size[e]; i += kSlots * kTileThreads) {
+      for (int i = first + wave0; i < end; i += kSlots * kTileThreads) {
         uint4 acc[kSlots];
         int at[kSlots];
 #pragma unroll
-        for (int u = 0; u < kSlots; u++) at[u] = min(i + lane + u * kTileThreads, 2 * size[e] - 1);
-        const uint4* in = above(0);
+        for (int u = 0; u < kSlots; u++) at[u] = min(i + lane + u * kTileThreads, end - 1);
+        const uint4* in = entry(word(up));
 #pragma unroll
         for (int u = 0; u < kSlots; u++) acc[u] = in[at[u]];
         int j = 1;
@@ -188,7 +175,7 @@ __device__ __forceinline__ void mid_tile(const TileJob& J, const MidTabs& M, int
           uint4 x[kAbove][kSlots];
 #pragma unroll
           for (int k = 0; k < kAbove; k++) {
-            const uint4* in = above(j + k);
+            const uint4* in = entry(word(up + j + k));
 #pragma unroll
             for (int u = 0; u < kSlots; u++) x[k][u] = in[at[u]];
           }
@@ -198,7 +185,7 @@ __device__ __forceinline__ void mid_tile(const TileJob& J, const MidTabs& M, int
             for (int u = 0; u < kSlots; u++) or4(acc[u], x[k][u]);
         }
         for (; j < nhigh; j++) {
-          const uint4* in = above(j);
+          const uint4* in = entry(word(up + j));
 #pragma unroll
           for (int u = 0; u < kSlots; u++) or4(acc[u], in[at[u]]);
         }
@@ -206,75 +193,67 @@ __device__ __forceinline__ void mid_tile(const TileJob& J, const MidTabs& M, int
         for (int u = 0; u < kSlots; u++) lds.half[(e ? 2 * size[0] : 0) + at[u]] = acc[u];
       }
     }
-  const uint4 none = make_uint4(0, 0, 0, 0);
-  MidClass c = get_class(low);
-  Kids kids, ahead;
-  if (wave0 < c.count()) kids = M.kids[2 * c.members() + ((h + low) & 1) * c.count() + min(tid, c.count() - 1)];
-  const uint4* kid_half = nullptr;   // class l + 1
-  int kid_count = 0;
-  for (int l = low; l >= 0; l--) {
-    const int n = h + l, mover = n & 1, par = (n + J.ply) & 1;
-    const MidClass cn = get_class(l - 1);
-    if (wave0 < cn.count())
-      ahead = M.kids[2 * cn.members() + ((h + l - 1) & 1) * cn.count() + min(tid, cn.count() - 1)];
-    uint4* half = lds.half + 2 * ((l & 1 ? size[0] : 0) + c.at());
-    tile_barrier();   // the tiles above (first round) or class l + 1 are in the LDS
-    if (wave0 < c.count()) {
-      const int r = min(tid, c.count() - 1);
-      Two acc = {none, none};
-      if (nhigh) acc = Two{half[r], half[c.count() + r]};
-      if (n == spots) acc.nl = make_uint4(~0u, ~0u, ~0u, ~0u);   // the board is full: not lost
-      auto kid = [&](uint32_t rank16) {
-        const char* in = reinterpret_cast<const char*>(kid_half) + rank16;
-        return Two{*reinterpret_cast<const uint4*>(in), *reinterpret_cast<const uint4*>(in + 16 * kid_count)};
-      };
+  // first slots of the classes from the highest on, below the class's own chain 0
+  int at[2] = {size[0], size[1]};
+  const uint4* kid_half = nullptr;   // class l + 1, chain 0
 #pragma unroll
-      for (int j = 0; j < kTileCells; j += 2) {
-        if (j + 1 < kTileCells && j + 1 < low - l)
-          or_two(acc, kid(kids.rank16[j]), kid(kids.rank16[j + 1]));
-        else if (j < low - l)
-          or_two(acc, kid(kids.rank16[j]));
-      }
-      const uint32_t A = kids.mem & 0xff, Bm = kids.mem >> 8;
+  for (int l = kTileCells; l >= 0; l--) {
+    if (l > low) continue;
+    const int n = h + l, mover = n & 1, par = (n + J.ply) & 1, e = l & 1, c = count(l);
+    at[e] -= c;
+    uint4* half = lds.half + (e ? 2 * size[0] : 0) + at[e];
+    tile_barrier();   // the tiles above (first round) or class l + 1 are in the LDS
+    if (wave0 < c) {
+      const int r = min(t, c - 1);
+      const uint32_t mem = l ? kids[l].w[1] >> 16 : 0, A = mem & 0xff, Bm = mem >> 8;
       const uint4 imm0 = lds.wins[mover][par][mover ? Bm : A];
       const uint4 after = lds.wins[mover ^ 1][par][mover ? A : Bm];
       const uint4 before = lds.wins[mover ^ 1][par ^ 1][mover ? A : Bm];
-      // The side to move wins at once (imm0) unless the other side has five too (after), else
-      // by a child; not lost likewise.  Of (children, imm0, after): win (c & ~(i | a)) | (i & ~a)
-      // = 0x54, not lost (c & ~(i | a)) | i = 0xDC; here their complements, whose hrmax,
-      // exchanged, is the other side's view, which the parents read.
-      uint4 lw, ln;
-      lw.x = lop3_32<0xAB>(acc.win.x, imm0.x, after.x); ln.x = lop3_32<0x23>(acc.nl.x, imm0.x, after.x);
-      lw.y = lop3_32<0xAB>(acc.win.y, imm0.y, after.y); ln.y = lop3_32<0x23>(acc.nl.y, imm0.y, after.y);
-      lw.z = lop3_32<0xAB>(acc.win.z, imm0.z, after.z); ln.z = lop3_32<0x23>(acc.nl.z, imm0.z, after.z);
-      lw.w = lop3_32<0xAB>(acc.win.w, imm0.w, after.w); ln.w = lop3_32<0x23>(acc.nl.w, imm0.w, after.w);
-      if (n <= 1 && tid < c.count()) {
-        const uint32_t root = p << low | A;
-        uint4* res = reinterpret_cast<uint4*>(&J.results[n ? 1 + __builtin_ctz(root) : 0]);
-        res[0] = make_uint4(~lw.x, ~lw.y, ~lw.z, ~lw.w);
-        res[1] = make_uint4(~ln.x, ~ln.y, ~ln.z, ~ln.w);
-      }
-      const uint4 sw = hrmax4(ln, before), sn = hrmax4(lw, before);
-      if (tid < c.count()) {
-        half[tid] = sw;
-        half[c.count() + tid] = sn;
-        const uint32_t to = n & 1 ? own.y : own.x;
-        if (to != kNotStored) {
-          uint4* out = reinterpret_cast<uint4*>(entry(to + uint32_t(c.at())));
-          if (J.stream) {
-            store_stream(&out[tid], sw);
-            store_stream(&out[c.count() + tid], sn);
-          } else {
-            out[tid] = sw;
-            out[c.count() + tid] = sn;
+      const uint32_t own = word(kRecOwn + mover);
+#pragma unroll
+      for (int k = 0; k < 3 - kChains; k++) {
+        const int chain = chain0 + k;
+        const bool notlose = (mover ^ chain) != 0;   // wave-uniform
+        uint4 acc = make_uint4(0, 0, 0, 0);
+        if (nhigh) acc = half[chain * size[e] + r];
+        if (n == spots && notlose) acc = make_uint4(~0u, ~0u, ~0u, ~0u);   // the board is full: not lost
+        auto kid = [&](int j) {
+          return kid_half[chain * size[e ^ 1] + int(kids[l].w[j >> 2] >> (8 * (j & 3)) & 0xff)];
+        };
+#pragma unroll
+        for (int j = 0; j < kTileCells - l; j += 2) {
+          if (j + 1 < low - l) or4(acc, kid(j), kid(j + 1));
+          else if (j < low - l) or4(acc, kid(j));
+        }
+        // The side to move wins at once (imm0) unless the other side has five too (after), else
+        // by a child; not lost likewise.  Of (children, imm0, after): win (c & ~(i | a)) | (i & ~a)
+        // = 0x54, not lost (c & ~(i | a)) | i = 0xDC; here their complements, whose hrmax is the
+        // other side's view, which the parents read.
+        uint4 x;
+        if (notlose) {
+          x.x = lop3_32<0x23>(acc.x, imm0.x, after.x); x.y = lop3_32<0x23>(acc.y, imm0.y, after.y);
+          x.z = lop3_32<0x23>(acc.z, imm0.z, after.z); x.w = lop3_32<0x23>(acc.w, imm0.w, after.w);
+        } else {
+          x.x = lop3_32<0xAB>(acc.x, imm0.x, after.x); x.y = lop3_32<0xAB>(acc.y, imm0.y, after.y);
+          x.z = lop3_32<0xAB>(acc.z, imm0.z, after.z); x.w = lop3_32<0xAB>(acc.w, imm0.w, after.w);
+        }
+        if (n <= 1 && t < c) {
+          const uint32_t root = p << low | A;
+          uint4* res = reinterpret_cast<uint4*>(&J.results[n ? 1 + __builtin_ctz(root) : 0]);
+          res[notlose] = make_uint4(~x.x, ~x.y, ~x.z, ~x.w);
+        }
+        x = hrmax4(x, before);
+        if (t < c) {
+          half[chain * size[e] + t] = x;
+          if (own != kNotStored) {
+            uint4* out = entry(own) + (chain * size[e] + at[e]);
+            if (J.stream) store_stream(&out[t], x);
+            else out[t] = x;
           }
         }
       }
     }
     kid_half = half;
-    kid_count = c.count();
-    c = cn;
-    kids = ahead;
   }
 }
 

@@ -37,27 +37,47 @@ __global__ __launch_bounds__(256) void mid_prep_kernel(const MidBoardDev* __rest
   mid_wins_entry(boards[b], t - prefix[b], T);
 }
 
-// Step `step` of every board that has one: workgroup w sweeps tile w - prefix[b] of the
-// step's tiles of board b.
+// One board's table, by value.
+__global__ __launch_bounds__(256) void mid_prep_one_kernel(MidBoardDev B, int64_t total, DevTables T) {
+  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  if (t < total) mid_wins_entry(B, t, T);
+}
+
 // Workgroup i runs on XCD i % 8: each XCD takes runs of neighbouring tiles, which read the same
 // tiles.  Runs of 1 / 4 / 16 / 64 tiles measured within 3 %, 16 the fastest; one run of an eighth
 // of the launch to each XCD is 20 % slower (the groups of a step differ in tile size).
 constexpr int kRun = 16;
+__device__ __forceinline__ int run_order() {
+  const int x = blockIdx.x & 7, y = blockIdx.x >> 3;
+  return (y / kRun * 8 + x) * kRun + y % kRun;
+}
+unsigned run_grid(int64_t tiles) { return unsigned((tiles + 8 * kRun - 1) / (8 * kRun) * (8 * kRun)); }
 // A step that writes more than this (24 KB a tile at most) than the L2s hold together, 32 MB, is
 // stored past them: 18 empty cells 2.51 -> 2.43 ms; a small step's reader finds it in the L2.
 constexpr int kStreamTiles = 2048;
+
+// Step `step` of every board that has one: workgroup w sweeps tile w - prefix[b] of the
+// step's tiles of board b.
 __global__ __launch_bounds__(kTileThreads, 5) void mid_step_kernel(const MidBoardDev* __restrict__ boards,
                                                                 const int64_t* __restrict__ prefix, int nb,
-                                                                int step, int ntiles, MidTabs M) {
+                                                                int step, int ntiles, MidTabsDev M) {
   __shared__ TileLds lds;
-  const int x = blockIdx.x & 7, y = blockIdx.x >> 3;
-  const int w = (y / kRun * 8 + x) * kRun + y % kRun;
+  const int w = run_order();
   if (w >= ntiles) return;
-  const int b = nb == 1 ? 0 : find_board(prefix, nb, w);
-  const int t = w - (nb == 1 ? 0 : int(prefix[b]));
+  const int b = find_board(prefix, nb, w);
+  const int t = w - int(prefix[b]);
   const MidBoardDev& B = boards[b];
   const MidSched& S = M.sched[B.I.spots];
-  mid_tile(tile_job(B, B.work, S, M, ntiles > kStreamTiles), M, S.first[step] + t, lds, int(threadIdx.x));
+  mid_tile<1>(tile_job(B, B.work, S, M, ntiles > kStreamTiles), S.first[step] + t, lds, int(threadIdx.x));
+}
+
+// A step of one board, by value: `ntiles` tiles from `first` on.
+template <int kChains>
+__global__ __launch_bounds__(kTileThreads * kChains, kChains == 2 ? 4 : 5) void mid_step_one_kernel(TileJob J, int first,
+                                                                                                  int ntiles) {
+  __shared__ TileLds lds;
+  const int w = run_order();
+  if (w < ntiles) mid_tile<kChains>(J, first + w, lds, int(threadIdx.x));
 }
 
 }  // namespace
@@ -89,13 +109,28 @@ void mid_carve(MidBoardDev* B, uint8_t* base) {
   B->results = reinterpret_cast<pe_halfsupers*>(base + t + mid_work_bytes(B->I));
 }
 
-pe_status mid_launch_step(const MidBoardDev* board, const MidInfo& info, int step, const DevTables& T,
-                          hipStream_t stream) {
-  const int64_t tiles = mid_step_tiles(info, step);
-  if (tiles <= 0) return PE_OK;
-  hipLaunchKernelGGL(mid_step_kernel, dim3(unsigned((tiles + 8 * kRun - 1) / (8 * kRun) * (8 * kRun))), dim3(kTileThreads), 0, stream, board, nullptr, 1, step,
-                     int(tiles), T.mid);
-  PE_HIP(hipGetLastError(), "mid_step_kernel launch");
+// Up to this many tiles a step's time is a tile's latency more than the chip's rate (1280 tiles
+// of 32 KB LDS are in flight at once): a thread for each chain of a tile, twice the waves.  One
+// MI355X, never / up to 512 / up to 4096 tiles: 26 stones 71.8 / 61.4 / 61.3 us, 22 stones 175 /
+// 161 / 158, 19 stones 917 / 914 / 905.
+constexpr int64_t kTwoChains = 4096;
+
+pe_status mid_launch_board(const MidBoardDev& B, const DevTables& T, hipStream_t stream) {
+  const int64_t total = mid_prep_entries(B.I);
+  hipLaunchKernelGGL(mid_prep_one_kernel, dim3(unsigned((total + 255) / 256)), dim3(256), 0, stream, B, total, T);
+  PE_HIP(hipGetLastError(), "mid_prep_one_kernel launch");
+  const MidSched& S = mid_tabs().sched[size_t(B.I.spots)];
+  for (int k = 0; k < S.steps; k++) {
+    const int64_t tiles = mid_step_tiles(B.I, k);
+    if (tiles <= 0) continue;
+    const TileJob J = tile_job(B, B.work, S, T.mid, tiles > kStreamTiles);
+    const dim3 grid(run_grid(tiles));
+    if (tiles <= kTwoChains)
+      hipLaunchKernelGGL(mid_step_one_kernel<2>, grid, dim3(2 * kTileThreads), 0, stream, J, S.first[k], int(tiles));
+    else
+      hipLaunchKernelGGL(mid_step_one_kernel<1>, grid, dim3(kTileThreads), 0, stream, J, S.first[k], int(tiles));
+    PE_HIP(hipGetLastError(), "mid_step_one_kernel launch");
+  }
   return PE_OK;
 }
 
@@ -118,6 +153,13 @@ pe_status mid_solve_levels(const std::vector<MidInfo>& infos, uint8_t* arena, st
   if (device_tables(&T, &err) != PE_OK) { set_error(err); return PE_ERR_DEVICE; }
   const int nb = int(infos.size());
   if (!nb) return PE_OK;
+  if (nb == 1) {
+    MidBoardDev B{};
+    B.I = infos[0];
+    mid_carve(&B, arena);
+    result_offsets->assign(1, size_t(reinterpret_cast<uint8_t*>(B.results) - arena));
+    return mid_launch_board(B, T, stream);
+  }
   std::vector<MidBoardDev> boards(nb);
   result_offsets->resize(nb);
   size_t off = 0;
@@ -163,7 +205,7 @@ pe_status mid_solve_levels(const std::vector<MidInfo>& infos, uint8_t* arena, st
     const int64_t total = p[nb];
     if (total <= 0) continue;
     if (total > 0x7fff0000) { set_error("too many tiles in one midsolve launch"); return PE_ERR_CAPACITY; }
-    hipLaunchKernelGGL(mid_step_kernel, dim3(unsigned((total + 8 * kRun - 1) / (8 * kRun) * (8 * kRun))), dim3(kTileThreads), 0, stream, dboards,
+    hipLaunchKernelGGL(mid_step_kernel, dim3(run_grid(total)), dim3(kTileThreads), 0, stream, dboards,
                        dprefix + size_t(nb + 1) * (t + 1), nb, t, int(total), T.mid);
     PE_HIP(hipGetLastError(), "mid_step_kernel launch");
   }
@@ -174,8 +216,7 @@ pe_status mid_solve_levels(const std::vector<MidInfo>& infos, uint8_t* arena, st
 // ---- allocation-free single-board solve ----
 // For callers that cannot allocate device memory (code under HIP graph capture, tight
 // serving loops, harnesses that forbid hipMalloc); the reference has no counterpart (its
-// caller passes a workspace it owns).  The launch descriptors, the board's tables, its
-// workspace and its results live in `scratch`, a fixed array that every device the library
+// caller passes a workspace it owns).  The board's tables, its workspace and its results live in `scratch`, a fixed array that every device the library
 // runs on holds until the process ends.  Host code never uses the array's name as an
 // address: each device's address comes from hipGetSymbolAddress, once per device.
 constexpr size_t kScratchBytes = size_t(64) << 20;
@@ -186,13 +227,6 @@ namespace {
 constexpr int kScratchDevices = 64;
 std::mutex g_scratch_mu[kScratchDevices];      // one solve at a time per device in this process
 uint8_t* g_scratch_ptr[kScratchDevices];       // device address of `scratch` on each device
-
-// The descriptors of one board's launches: the board record, then the prefix the prep kernel
-// reads ([0, entries]).
-struct NoAllocDesc {
-  MidBoardDev board;
-  int64_t prefix[2];
-};
 
 }  // namespace
 
@@ -206,8 +240,7 @@ pe_status mid_solve_noalloc(const pe_high_board& hb, pe_halfsupers* results, hip
     set_error("the device's tables are not uploaded: call pe_init on this device first (this entry point allocates nothing)");
     return PE_ERR_INVALID;
   }
-  const size_t desc_bytes = align256(sizeof(NoAllocDesc));
-  const size_t need = desc_bytes + mid_board_bytes(I);
+  const size_t need = mid_board_bytes(I);
   if (need > kScratchBytes) {
     set_error("board with " + std::to_string(I.spots) + " empty cells needs " + std::to_string(need) +
               " bytes of device scratch; the allocation-free solve has " + std::to_string(kScratchBytes) +
@@ -226,24 +259,18 @@ pe_status mid_solve_noalloc(const pe_high_board& hb, pe_halfsupers* results, hip
   uint8_t* const base = g_scratch_ptr[dev];
   // every table, workspace and result entry the kernels read is written by them first
   // (prep, then the tile layers), so nothing in the array needs clearing between calls
-  NoAllocDesc d;
-  std::memset(&d, 0, sizeof d);
-  d.board.I = I;
-  mid_carve(&d.board, base + desc_bytes);
-  d.prefix[1] = mid_prep_entries(I);
-  // every way out waits for the work queued on the stream: the descriptors are read from
-  // this frame, and the next call (on any stream) reuses the array
+  MidBoardDev B{};
+  B.I = I;
+  mid_carve(&B, base);
+  // every way out waits for the work queued on the stream: the next call (on any stream) reuses
+  // the array
   struct Drain {
     hipStream_t s;
     ~Drain() { (void)hipStreamSynchronize(s); }
   } drain{stream};
-  PE_HIP(hipMemcpyAsync(base, &d, sizeof d, hipMemcpyHostToDevice, stream), "hipMemcpyAsync(descriptors)");
-  const auto* dboard = reinterpret_cast<const MidBoardDev*>(base);
-  const auto* dprefix = reinterpret_cast<const int64_t*>(base + offsetof(NoAllocDesc, prefix));
-  pe_status st = mid_launch_prep(dboard, dprefix, 1, d.prefix[1], T, stream);
-  for (int k = 0; k < mid_steps(I) && st == PE_OK; k++) st = mid_launch_step(dboard, I, k, T, stream);
+  const pe_status st = mid_launch_board(B, T, stream);
   if (st != PE_OK) return st;
-  PE_HIP(hipMemcpyAsync(results, d.board.results, sizeof(pe_halfsupers) * 19, hipMemcpyDeviceToHost, stream),
+  PE_HIP(hipMemcpyAsync(results, B.results, sizeof(pe_halfsupers) * 19, hipMemcpyDeviceToHost, stream),
          "hipMemcpyAsync(results)");
   PE_HIP(hipStreamSynchronize(stream), "allocation-free midsolve");
   for (int i = I.spots + 1; i < 19; i++) std::memset(&results[i], 0, sizeof(pe_halfsupers));

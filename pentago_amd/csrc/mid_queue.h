@@ -18,7 +18,14 @@
 
 namespace pe {
 
-struct MidBoardDev;
+// A board's descriptor: what its kernels read and write.
+struct MidBoardDev {
+  MidInfo I;
+  uint64_t* wins;           // [mover of the root, other][mask of empty cells]: halves of parity 0, 1
+  uint64_t* spill;          // tile entries that the workspace has no room for
+  uint64_t* work;           // tile entries, 4 u64 each
+  pe_halfsupers* results;   // 19 entries
+};
 
 struct MidConfig {
   int64_t budget;        // bytes one run may hold (tables, workspaces, descriptors)
@@ -39,7 +46,8 @@ struct MidLayout {
   size_t small_work = 0, small_stride = 0;   // workspace slot of each workgroup
   size_t big_slots = 0, big_stride = 0;      // per stream: tables, then workspace
   size_t bytes = 0;                    // total
-  // descriptor blob at offset 0: small boards | big boards | prep prefixes | results | head
+  // descriptor blob at offset 0: small boards | big boards | prep prefixes | results | head (the
+  // large boards' share is part of the reported bytes only: their launches take them by value)
   size_t o_big = 0, o_prefix = 0, o_res = 0, o_head = 0, blob_bytes = 0;
 };
 // Returns null on success, else an error message.
@@ -58,12 +66,11 @@ struct MidPlan {
   bool captured = false;               // a run was captured: nobody knows when the memory is free
   bool owns_mem = true;                // false: caller memory, not freed by the plan
   const MidBoardDev* small_dev = nullptr;
-  const MidBoardDev* big_dev = nullptr;
-  const int64_t* prefix = nullptr;     // small boards' prep prefix, then [0, total] per big board
+  std::vector<MidBoardDev> big;        // large boards: launches take them by value
+  const int64_t* prefix = nullptr;     // small boards' prep prefix
   pe_halfsupers* results = nullptr;    // 19 per board, in board order
   unsigned int* head = nullptr;
   int64_t small_prep_total = 0;
-  std::vector<int64_t> big_prep_total;
   DevTables tables{};
   std::vector<hipStream_t> streams;    // owned, layout.streams of them
   std::vector<hipEvent_t> events;      // fork + one join per stream
@@ -114,8 +121,7 @@ pe_status mid_launch_prep(const MidBoardDev* boards, const int64_t* prefix, int 
 inline int64_t mid_prep_entries(const MidInfo& I) { return int64_t(2) << I.spots; }
 int mid_steps(const MidInfo& I);
 int64_t mid_step_tiles(const MidInfo& I, int step);
-// One launch sweeping the tiles of one step of one board.
-pe_status mid_launch_step(const MidBoardDev* board, const MidInfo& info, int step, const DevTables& T,
-                          hipStream_t stream);
+// Every launch of one board, its descriptor passed by value.
+pe_status mid_launch_board(const MidBoardDev& board, const DevTables& T, hipStream_t stream);
 
 }  // namespace pe

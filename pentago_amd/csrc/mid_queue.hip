@@ -23,7 +23,7 @@ __global__ void mid_head_reset_kernel(unsigned int* head) { *head = 0; }
 template <int kThreads>
 __global__ __launch_bounds__(kThreads, 4) void mid_boards_kernel(const MidBoardDev* __restrict__ boards, int nboards,
                                                                  uint8_t* __restrict__ work_base, int64_t work_stride,
-                                                                 unsigned int* __restrict__ head, MidTabs M) {
+                                                                 unsigned int* __restrict__ head, MidTabsDev M) {
   constexpr int kSub = kThreads / kTileThreads;
   __shared__ TileLds lds[kSub];
   __shared__ int s_b;
@@ -40,7 +40,7 @@ __global__ __launch_bounds__(kThreads, 4) void mid_boards_kernel(const MidBoardD
     const TileJob J = tile_job(B, work, S, M, false);
     for (int k = 0; k < S.steps; k++) {
       for (int t = S.first[k]; t < S.first[k + 1]; t += kSub) {
-        mid_tile(J, M, t + sub < S.first[k + 1] ? t + sub : -1, lds[sub], int(threadIdx.x) % kTileThreads);
+        mid_tile<1>(J, t + sub < S.first[k + 1] ? t + sub : -1, lds[sub], int(threadIdx.x) % kTileThreads);
         tile_barrier();   // before the next tile's wins replace this one's
       }
       __syncthreads();
@@ -145,7 +145,6 @@ pe_status mid_plan_create(const std::vector<MidInfo>& infos, const MidConfig& cf
   // descriptors
   std::vector<uint8_t> blob(L.o_res, 0);
   auto* sdev = reinterpret_cast<MidBoardDev*>(blob.data());
-  auto* bdev = reinterpret_cast<MidBoardDev*>(blob.data() + L.o_big);
   auto* prefix = reinterpret_cast<int64_t*>(blob.data() + L.o_prefix);
   auto* res = reinterpret_cast<pe_halfsupers*>(base + L.o_res);
   prefix[0] = 0;
@@ -160,20 +159,15 @@ pe_status mid_plan_create(const std::vector<MidInfo>& infos, const MidConfig& cf
     prefix[k + 1] = prefix[k] + mid_prep_entries(B.I);
   }
   plan->small_prep_total = prefix[L.small.size()];
-  plan->big_prep_total.resize(L.big.size());
+  plan->big.resize(L.big.size());
   for (size_t k = 0; k < L.big.size(); k++) {
-    MidBoardDev B;
+    MidBoardDev& B = plan->big[k];
     std::memset(&B, 0, sizeof B);
     B.I = infos[size_t(L.big[k])];
     uint8_t* slot = base + L.big_slots + size_t(L.big_stream[k]) * L.big_stride;
     mid_carve_tables(&B, slot);
     B.work = reinterpret_cast<uint64_t*>(slot + mid_table_bytes(B.I));
     B.results = res + 19 * size_t(L.big[k]);
-    std::memcpy(&bdev[k], &B, sizeof B);
-    int64_t* p = prefix + L.small.size() + 1 + 2 * k;
-    p[0] = 0;
-    p[1] = mid_prep_entries(B.I);
-    plan->big_prep_total[k] = p[1];
   }
   if (alloc_stream && upload && blob.size() <= upload_bytes) {
     // pinned staging owned by the caller: the copy is queued, nothing waits
@@ -189,7 +183,6 @@ pe_status mid_plan_create(const std::vector<MidInfo>& infos, const MidConfig& cf
   }
   if (plan->mem_cap) PE_HIP(hipEventCreateWithFlags(&plan->done, hipEventDisableTiming), "hipEventCreate(mid batch)");
   plan->small_dev = reinterpret_cast<const MidBoardDev*>(base);
-  plan->big_dev = reinterpret_cast<const MidBoardDev*>(base + L.o_big);
   plan->prefix = reinterpret_cast<const int64_t*>(base + L.o_prefix);
   plan->results = res;
   plan->head = reinterpret_cast<unsigned int*>(base + L.o_head);
@@ -240,32 +233,19 @@ pe_status launch_small(const MidPlan& plan, hipStream_t s) {
   return PE_OK;
 }
 
-pe_status launch_big(const MidPlan& plan, size_t k, hipStream_t s) {
-  const MidLayout& L = plan.layout;
-  const MidInfo& I = plan.infos[size_t(L.big[k])];
-  const MidBoardDev* B = plan.big_dev + k;
-  pe_status st = mid_launch_prep(B, plan.prefix + L.small.size() + 1 + 2 * k, 1, plan.big_prep_total[k], plan.tables, s);
-  if (st != PE_OK) return st;
-  for (int n = 0; n < mid_steps(I); n++) {
-    st = mid_launch_step(B, I, n, plan.tables, s);
-    if (st != PE_OK) return st;
-  }
-  return PE_OK;
-}
-
 // The whole run on `stream`, forking the large boards onto the plan's streams.
 pe_status launch_all(const MidPlan& plan, hipStream_t stream) {
   const MidLayout& L = plan.layout;
   if (L.streams == 0) {
     pe_status st = launch_small(plan, stream);
-    for (size_t k = 0; k < L.big.size() && st == PE_OK; k++) st = launch_big(plan, k, stream);
+    for (size_t k = 0; k < L.big.size() && st == PE_OK; k++) st = mid_launch_board(plan.big[k], plan.tables, stream);
     return st;
   }
   PE_HIP(hipEventRecord(plan.events[0], stream), "hipEventRecord(fork)");
   for (int s = 0; s < L.streams; s++)
     PE_HIP(hipStreamWaitEvent(plan.streams[size_t(s)], plan.events[0], 0), "hipStreamWaitEvent(fork)");
   for (size_t k = 0; k < L.big.size(); k++) {
-    const pe_status st = launch_big(plan, k, plan.streams[size_t(L.big_stream[k])]);
+    const pe_status st = mid_launch_board(plan.big[k], plan.tables, plan.streams[size_t(L.big_stream[k])]);
     if (st != PE_OK) return st;
   }
   const pe_status st = launch_small(plan, stream);

@@ -227,6 +227,50 @@ MidTabs MidTabsHost::view() const {
   return MidTabs{sched.data(), tiles.data(), bases.data(), classes.data(), kids.data()};
 }
 
+std::vector<uint32_t> mid_records(const MidTabs& M) {
+  std::vector<uint32_t> out;
+  for (int spots = 0; spots <= kMidSpots; spots++) {
+    const MidSched& S = M.sched[spots];
+    for (int t = S.tiles; t < S.tiles + S.first[S.steps]; t++) {
+      const MidTile& X = M.tiles[t];
+      const int d = __builtin_popcount(X.p) - __builtin_popcount(X.q);
+      uint32_t r[kRecWords] = {};
+      r[0] = X.p | X.q << 16;
+      for (int par = 0; par < 2; par++) r[kRecOwn + par] = M.bases[2 * (size_t(S.bases) + X.code) + size_t(par)];
+      for (int l = 0; l <= S.low; l++) {
+        const uint32_t n = uint32_t(M.classes[mid_class_row(S.low, d, l)].count());
+        r[kRecSizes] += n << (l & 1 ? 16 : 0);
+        r[kRecCounts + l / 4] |= n << (8 * (l % 4));
+      }
+      uint32_t c3 = 1;
+      for (int c = 0, j = 0; c < S.high; c++, c3 *= 3) {
+        if ((X.p | X.q) >> c & 1) continue;
+        for (int m = 0; m < 2; m++)
+          r[kRecUp + m * kRecUp1 + j] = M.bases[2 * (size_t(S.bases) + X.code + (m + 1u) * c3) + (m ? 0 : 1)];
+        j++;
+      }
+      out.insert(out.end(), r, r + kRecWords);
+    }
+  }
+  return out;
+}
+
+std::vector<KidRanks> mid_kid_ranks(const MidTabs& M) {
+  std::vector<KidRanks> out(size_t(mid_kid_row(kTileCells + 1, -11, 0)), KidRanks{{0, 0}});
+  for (int low = 0; low <= kTileCells; low++)
+    for (int d = -11; d <= 11; d++)
+      for (int l = 0; l <= low; l++) {
+        const MidClass& c = M.classes[mid_class_row(low, d, l)];
+        for (int r = 0; r < c.count(); r++) {
+          const Kids& k = M.kids[2 * c.members() + ((d + l) & 1) * c.count() + r];
+          KidRanks& o = out[size_t(mid_kid_row(low, d, l) + r)];
+          o.w[1] = uint32_t(k.mem) << 16;
+          for (int j = 0; j < low - l; j++) o.w[j / 4] |= uint32_t(k.rank16[j] / 16) << (8 * (j % 4));
+        }
+      }
+  return out;
+}
+
 int64_t mid_work_entries(int spots) { return bottleneck(spots); }
 
 // Part of the plans' memory contract (pe_mid_schedule_info reports it, budgets are checked

@@ -59,7 +59,7 @@ struct MidClass {
 // inside the tile, by ascending cell, and A | B << 8.
 struct Kids { uint16_t rank16[kTileCells], mem; };
 
-// Lookup tables (host vectors or device pointers).
+// Lookup tables on the host.
 struct MidTabs {
   const MidSched* sched;             // [kMidSpots + 1]
   const MidTile* tiles;
@@ -76,6 +76,28 @@ struct MidTabsHost {
   MidTabs view() const;
 };
 constexpr int mid_class_row(int low, int d, int l) { return (low * 23 + d + 11) * 9 + l; }
+
+// The device's form of the tables, which a workgroup has in two dependent loads (the tile's
+// record, then everything that the record leads to).
+//
+// A tile's record is 32 words, one to a lane: p | q << 16; the first entries of its own halves
+// (even levels, odd levels); entries of its classes of even l | of odd l << 16; the classes'
+// counts, a byte each; and by empty high cell in ascending order the first entries of the halves
+// it may read there: the odd levels of the tile with the cell filled by M0, the even ones of the
+// tile with it filled by M1.
+constexpr int kRecWords = 32, kRecOwn = 1, kRecSizes = 3, kRecCounts = 4, kRecUp = 6, kRecUp1 = kMidSpots - kTileCells;
+// Ranks of a member's children by ascending cell, a byte each, and in the last two bytes its masks
+// A and B; the one member of class 0 (no stones) may have a seventh child, in the place of A.
+struct KidRanks { uint32_t w[2]; };
+// The mover of class l is (d + l) & 1 (d and a + b have one parity): a row of kTileClass members.
+constexpr int mid_kid_row(int low, int d, int l) { return ((low * 23 + d + 11) * (kTileCells + 1) + l) * kTileClass; }
+struct MidTabsDev {
+  const MidSched* sched;
+  const uint32_t* records;           // kRecWords a tile, in the order of MidTabs::tiles
+  const KidRanks* kids;              // [mid_kid_row + rank]
+};
+std::vector<uint32_t> mid_records(const MidTabs& M);
+std::vector<KidRanks> mid_kid_ranks(const MidTabs& M);
 
 // Entries (32 bytes) of a board's two areas: its workspace, and its table area, which holds
 // the wins tables (2 << spots entries) and then the spill area.

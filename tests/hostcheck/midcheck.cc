@@ -82,6 +82,47 @@ int mc_layout(int spots) {
   return faults + (positions != expect) + int(held.size());
 }
 
+// The records and child ranks that the device reads, against the tables: the number of words
+// that differ, of tiles and members whose low cells number mid_low_cells(spots).
+int mc_device_tables(int spots) {
+  const MidTabs M = mid_tabs().view();
+  const MidSched& S = M.sched[spots];
+  const std::vector<uint32_t> recs = mid_records(M);
+  const std::vector<KidRanks> ranks = mid_kid_ranks(M);
+  int faults = 0;
+  for (int t = S.tiles; t < S.tiles + S.first[S.steps]; t++) {
+    const uint32_t* r = recs.data() + size_t(kRecWords) * size_t(t);
+    const MidTile& X = M.tiles[t];
+    const int d = __builtin_popcount(X.p) - __builtin_popcount(X.q);
+    faults += (r[0] & 0xffff) != X.p || r[0] >> 16 != X.q;
+    for (int par = 0; par < 2; par++) faults += r[kRecOwn + par] != M.bases[2 * (S.bases + X.code) + par];
+    uint32_t size[2] = {0, 0};
+    for (int l = 0; l <= kTileCells; l++) {
+      const uint32_t n = l <= S.low ? uint32_t(M.classes[mid_class_row(S.low, d, l)].count()) : 0;
+      size[l & 1] += n;
+      faults += (r[kRecCounts + l / 4] >> (8 * (l % 4)) & 0xff) != n;
+    }
+    faults += r[kRecSizes] != (size[0] | size[1] << 16);
+    for (int c = 0, j = 0; c < S.high; c++)
+      if (!((X.p | X.q) >> c & 1)) {
+        faults += r[kRecUp + j] != M.bases[2 * (S.bases + X.code + pow3(c)) + 1];
+        faults += r[kRecUp + kRecUp1 + j] != M.bases[2 * (S.bases + X.code + 2 * pow3(c))];
+        j++;
+      }
+  }
+  for (int d = -11; d <= 11; d++)
+    for (int l = 0; l <= S.low; l++) {
+      const MidClass& c = M.classes[mid_class_row(S.low, d, l)];
+      for (int i = 0; i < c.count(); i++) {
+        const KidRanks& k = ranks[size_t(mid_kid_row(S.low, d, l) + i)];
+        const Kids& x = M.kids[2 * c.members() + ((d + l) & 1) * c.count() + i];
+        for (int j = 0; j < S.low - l; j++) faults += 16 * (k.w[j >> 2] >> (8 * (j & 3)) & 0xff) != x.rank16[j];
+        faults += l && k.w[1] >> 16 != x.mem;
+      }
+    }
+  return faults;
+}
+
 // One board solved on the CPU, as mid_tile does; 0 on success.
 int mc_solve(uint64_t side0, uint64_t side1, uint32_t ply, uint64_t* results) {
   pe_high_board hb{{side0, side1}, ply};

@@ -30,6 +30,11 @@ def test_tiles_are_stored_until_read(mc, spots):
     assert mc.mc_layout(spots) == 0
 
 
+@pytest.mark.parametrize("spots", [0, 1, 6, 7, 8, 13, 18])
+def test_device_tables(mc, spots):
+    assert mc.mc_device_tables(spots) == 0
+
+
 @pytest.mark.parametrize("stones", [24, 25, 26, 27, 28, 29, 34, 35, 36])
 def test_tile_sweep_matches_oracle(mc, stones):
     rng = np.random.default_rng(stones)
