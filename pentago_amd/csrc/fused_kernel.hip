@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <array>
 #include <atomic>
 #include <cstring>
 #include <map>
@@ -563,6 +564,74 @@ struct SlabBuild {
   std::string err;
 };
 
+// Where two dimensions' lines standardize to one child section along one child dimension (the
+// section maps to itself under a rotation of the board), block b's line along the one and block
+// b2's along the other read the same child nodes when b2 is b with its coordinates permuted:
+// b2[m[a]] = b[a].  The permutations of one slab's section, by its first lines.
+static std::vector<std::array<int, 4>> line_symmetries(const std::vector<const LineHost*>& first) {
+  std::vector<std::array<int, 4>> out;
+  for (size_t i = 0; i < first.size(); i++)
+    for (size_t j = 0; j < first.size(); j++) {
+      const pe_line_info &x = first[i]->info, &y = first[j]->info;
+      if (i == j || first[i]->dev.slice35 || x.child_dimension != y.child_dimension ||
+          (x.section_transform & 4) != (y.section_transform & 4) || !same_section(x.standard_child, y.standard_child))
+        continue;
+      std::array<int, 4> m;
+      for (int c = 0; c < 4; c++) m[size_t(x.permutation[c])] = y.permutation[c];
+      out.push_back(m);
+    }
+  return out;
+}
+
+// The order of a box's blocks: `order` lists them as numbers over the box (C order over
+// `extent`), and blocks that read the same children (line_symmetries) are brought together:
+// eight blocks, then what shares with each of them, eight apart, so that workgroups of
+// one XCD read the shared lines through one L2.
+constexpr size_t kTogether = 8;
+static void order_by_symmetry(const std::vector<std::array<int, 4>>& sym, const int lo[4], const int extent[4],
+                              std::vector<int64_t>* order) {
+  if (sym.empty()) return;
+  std::vector<char> placed(order->size(), 0);
+  std::vector<int64_t> out;
+  out.reserve(order->size());
+  std::vector<std::vector<int64_t>> group;
+  auto flush = [&]() {
+    for (size_t j = 0, any = 1; any; j++) {
+      any = 0;
+      for (const auto& g : group)
+        if (j < g.size()) { out.push_back(g[j]); any = 1; }
+    }
+    group.clear();
+  };
+  for (int64_t t : *order) {
+    if (placed[size_t(t)]) continue;
+    placed[size_t(t)] = 1;
+    std::vector<int64_t> orbit{t};
+    for (size_t k = 0; k < orbit.size(); k++) {
+      int b[4];
+      int64_t rest = orbit[k];
+      for (int a = 3; a >= 0; a--) {
+        b[a] = lo[a] + int(rest % extent[a]);
+        rest /= extent[a];
+      }
+      for (const auto& m : sym) {
+        int c[4];
+        for (int a = 0; a < 4; a++) c[m[size_t(a)]] = b[a];
+        int64_t u = 0;
+        for (int a = 0; a < 4 && u >= 0; a++)
+          u = c[a] < lo[a] || c[a] >= lo[a] + extent[a] ? -1 : u * extent[a] + (c[a] - lo[a]);
+        if (u < 0 || placed[size_t(u)]) continue;
+        placed[size_t(u)] = 1;
+        orbit.push_back(u);
+      }
+    }
+    group.push_back(std::move(orbit));
+    if (group.size() == kTogether) flush();
+  }
+  flush();
+  order->swap(out);
+}
+
 static void build_slab_body(const pe_slab& out, int nch, const pe_slab* ch, uint32_t dims, int accumulate,
                             SlabBuild* r) {
   const auto& Tb = tables();
@@ -598,14 +667,32 @@ static void build_slab_body(const pe_slab& out, int nch, const pe_slab* ch, uint
     if (a != inner) ord[nord++] = a;
   ord[3] = inner;
   int64_t total = 1;
-  for (int a = 0; a < 4; a++) total *= std::max(0, out.hi[a] - out.lo[a]);
-  int b[4];
+  int lo[4], extent[4], b[4];
+  for (int a = 0; a < 4; a++) {
+    lo[a] = out.lo[a];
+    extent[a] = std::max(0, out.hi[a] - out.lo[a]);
+    total *= extent[a];
+  }
+  std::vector<int64_t> order(static_cast<size_t>(total));
   for (int64_t t = 0; t < total; t++) {
-    int64_t rest = t;
+    int64_t rest = t, u = 0;
     for (int j = 3; j >= 0; j--) {
-      const int a = ord[j], e = out.hi[a] - out.lo[a];
-      b[a] = out.lo[a] + int(rest % e);
-      rest /= e;
+      b[ord[j]] = int(rest % extent[ord[j]]);
+      rest /= extent[ord[j]];
+    }
+    for (int a = 0; a < 4; a++) u = u * extent[a] + b[a];
+    order[size_t(t)] = u;
+  }
+  std::vector<const LineHost*> first;
+  for (int d = 0; d < 4; d++)
+    for (const LineHost& h : r->lines)
+      if (h.dev.dim == d) { first.push_back(&h); break; }
+  order_by_symmetry(line_symmetries(first), lo, extent, &order);
+  for (int64_t t : order) {
+    int64_t rest = t;
+    for (int a = 3; a >= 0; a--) {
+      b[a] = lo[a] + int(rest % extent[a]);
+      rest /= extent[a];
     }
     BlockDev B;
     B.sec = 0;
