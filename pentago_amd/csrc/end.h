@@ -107,7 +107,7 @@ struct BlockDev {
 
 struct FusedPlan {
   void* blob = nullptr;
-  int nblocks = 0;
+  int nblocks = 0, nfull = 0; // blocks from nfull on are ragged (the kernel's form for them)
   bool s35 = false;   // blocks of 35-stone sections (the kernel's no-children form)
   size_t off_lines = 0, off_secs = 0, off_moves = 0, off_refl = 0, off_heads = 0;
   int queue_wgs_per_cu = 0;   // 0: one workgroup per (block, part); else persistent queue form

@@ -48,20 +48,22 @@ namespace {
 enum { FH = 0, FV = 1, FLO = 2, FHI = 3, FAS = 4 };
 
 // Field words of one node: word k of field f of table t (0: F0, 1: F1, 2: Fm), quadrant q.
-// Quadrants 0 and 1 are read from global memory (the same entry for the whole wave),
-// quadrants 2 and 3 from the block's copy of its eight entries in LDS.
+// Quadrants 0 to kU - 1 are read from global memory (the same entry for the whole wave), the
+// others from the block's copy of their eight entries in LDS.
+template <int kU>
 struct NodeFields {
-  const uint64_t* glob[2];
-  const uint64_t* lds[2];
+  const uint64_t* glob[kU];
+  const uint64_t* lds[4 - kU];
   __device__ __forceinline__ uint64_t w(int q, int k, int t, int f) const {
-    return q < 2 ? glob[q][15 * k + 5 * t + f] : lds[q - 2][15 * k + 5 * t + f];
+    return q < kU ? glob[q][15 * k + 5 * t + f] : lds[q - kU][15 * k + 5 * t + f];
   }
 };
 
 // Word k of a pattern-group term for the three quantities: x[0] mover's side, x[1] other
 // side, x[2] the mover's side with one quadrant's field replaced by its OR over that
 // quadrant's moves (all moves at once).
-__device__ __forceinline__ void g2(const NodeFields& F, int k, int a, int fa, int b, int fb, uint64_t x[3]) {
+template <int kU>
+__device__ __forceinline__ void g2(const NodeFields<kU>& F, int k, int a, int fa, int b, int fb, uint64_t x[3]) {
   const uint64_t a0 = F.w(a, k, 0, fa), b0 = F.w(b, k, 0, fb);
   x[0] = a0 & b0;
   x[1] = F.w(a, k, 1, fa) & F.w(b, k, 1, fb);
@@ -70,23 +72,26 @@ __device__ __forceinline__ void g2(const NodeFields& F, int k, int a, int fa, in
 // The same terms with three-input logic operations (at least one of the quadrants is lane-
 // varying; products of two wave-uniform quadrants stay scalar).  g2_acc ORs the term into
 // acc; g2_term / g3_term return it.
-__device__ __forceinline__ void g2_acc(const NodeFields& F, int k, int a, int fa, int b, int fb, uint64_t acc[3]) {
+template <int kU>
+__device__ __forceinline__ void g2_acc(const NodeFields<kU>& F, int k, int a, int fa, int b, int fb, uint64_t acc[3]) {
   const uint64_t a0 = F.w(a, k, 0, fa), b0 = F.w(b, k, 0, fb);
   acc[0] = lop3<kOrAnd>(acc[0], a0, b0);
   acc[1] = lop3<kOrAnd>(acc[1], F.w(a, k, 1, fa), F.w(b, k, 1, fb));
   acc[2] = lop3<kOrAnd>(lop3<kOrAnd>(acc[2], F.w(a, k, 2, fa), b0), a0, F.w(b, k, 2, fb));
 }
-__device__ __forceinline__ void g2_term(const NodeFields& F, int k, int a, int fa, int b, int fb, uint64_t x[3]) {
+template <int kU>
+__device__ __forceinline__ void g2_term(const NodeFields<kU>& F, int k, int a, int fa, int b, int fb, uint64_t x[3]) {
   const uint64_t a0 = F.w(a, k, 0, fa), b0 = F.w(b, k, 0, fb);
   x[0] = a0 & b0;
   x[1] = F.w(a, k, 1, fa) & F.w(b, k, 1, fb);
   x[2] = lop3<kOrAnd>(F.w(a, k, 2, fa) & b0, a0, F.w(b, k, 2, fb));
 }
-// a2 b0 c0 | a0 b2 c0 | a0 b0 c2, with a (and b when b < 2) wave-uniform
-__device__ __forceinline__ void g3_term(const NodeFields& F, int k, int a, int fa, int b, int fb, int c, int fc,
+// a2 b0 c0 | a0 b2 c0 | a0 b0 c2, products of two wave-uniform quadrants first
+template <int kU>
+__device__ __forceinline__ void g3_term(const NodeFields<kU>& F, int k, int a, int fa, int b, int fb, int c, int fc,
                                         uint64_t x[3]) {
   const uint64_t a0 = F.w(a, k, 0, fa), b0 = F.w(b, k, 0, fb), c0 = F.w(c, k, 0, fc);
-  if (b < 2) {
+  if (a < kU && b < kU) {
     const uint64_t ab0 = a0 & b0, ab2 = (F.w(a, k, 2, fa) & b0) | (a0 & F.w(b, k, 2, fb));
     x[0] = ab0 & c0;
     x[1] = (F.w(a, k, 1, fa) & F.w(b, k, 1, fb)) & F.w(c, k, 1, fc);
@@ -118,15 +123,16 @@ constexpr int kWaves = 5;
 // One output block of 4096 nodes, computed by 16 workgroups (`part` = which 256 nodes).
 // S35: blocks of 35-stone sections, whose one move fills the board (no child data).
 // B.line[d] indexes `lines` for every open dimension d (-1: closed or not computed).
-template <bool S35>
+//
+// kU = 2: wave w of the block holds (loc0, loc1) = (w / 8, w % 8) and its 64 lanes (loc2, loc3):
+// quadrants 0 and 1 are the same for the whole wave, so their table reads are scalar loads and
+// their partial products scalar operations; lanes outside a partial edge block idle.
+// kU = 1: only quadrant 0 is, and the nodes of one loc0 fill waves in their stored order.
+template <bool S35, int kU>
 __device__ __forceinline__ void fused_block(const BlockDev& B, const SecDev& S, const LineDev* __restrict__ lines,
                                             const uint64_t* __restrict__ fields,
                                             const uint16_t* __restrict__ movetab, const uint8_t* __restrict__ refl,
                                             int part) {
-  // wave w of the block holds (loc0, loc1) = (w / 8, w % 8) and its 64 lanes (loc2, loc3):
-  // quadrants 0 and 1 are the same for the whole wave, so their table reads are scalar
-  // loads and their partial products scalar operations.  Lanes outside a partial edge
-  // block idle.
   const int wave = part * (kThreads / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
   // the block record's fields as plain int arrays (indexed by the dimension loop below)
@@ -139,21 +145,38 @@ __device__ __forceinline__ void fused_block(const BlockDev& B, const SecDev& S, 
   // the partial in the output slots, 3 finish from it (the result, stored)
   const int mode = B.accumulate;
   const bool partial_out = !S35 && (mode == 2 || mode == 4);
-  // the block's field entries of quadrants 2 and 3 (eight each) staged in LDS (the win
+  // the block's field entries of the other quadrants (eight each) staged in LDS (the win
   // patterns need them; a partial pass does not)
-  __shared__ uint64_t sf[2][8][60];
+  constexpr int kLane = 4 - kU;
+  __shared__ uint64_t sf[kLane][8][60];
   if (!partial_out) {   // uniform over the workgroup (one block)
-    for (int i = threadIdx.x; i < 2 * 8 * 60; i += kThreads) {
-      const int q = 2 + i / 480, r = (i / 60) % 8, w = i % 60;
-      const int bsq = q == 2 ? bs2 : bs3, bq = q == 2 ? bb[2] : bb[3];
-      const int64_t fo = q == 2 ? S.field_off[2] : S.field_off[3];
-      sf[q - 2][r][w] = r < bsq ? fields[4 * fo + 60 * int64_t(8 * bq + r) + w] : 0;
+    for (int i = threadIdx.x; i < kLane * 8 * 60; i += kThreads) {
+      const int x = i / 480, r = (i / 60) % 8, w = i % 60;
+      const int q = kU + x;
+      const int bsq = q == 1 ? bs1 : q == 2 ? bs2 : bs3, bq = q == 1 ? bb[1] : q == 2 ? bb[2] : bb[3];
+      const int64_t fo = q == 1 ? S.field_off[1] : q == 2 ? S.field_off[2] : S.field_off[3];
+      sf[x][r][w] = r < bsq ? fields[4 * fo + 60 * int64_t(8 * bq + r) + w] : 0;
     }
     __syncthreads();
   }
-  int loc[4] = {wave >> 3, wave & 7, lane >> 3, lane & 7};
-  if (loc[0] >= bs0 || loc[1] >= bs1 || loc[2] >= bs2 || loc[3] >= bs3) return;
-  const int p = ((loc[0] * bs1 + loc[1]) * bs2 + loc[2]) * bs3 + loc[3];
+  int loc[4], p;
+  if (kU == 2) {
+    loc[0] = wave >> 3, loc[1] = wave & 7, loc[2] = lane >> 3, loc[3] = lane & 7;
+    if (loc[0] >= bs0 || loc[1] >= bs1 || loc[2] >= bs2 || loc[3] >= bs3) return;
+    p = ((loc[0] * bs1 + loc[1]) * bs2 + loc[2]) * bs3 + loc[3];
+  } else {
+    const int n23 = bs2 * bs3, n123 = bs1 * n23, waves = (n123 + 63) >> 6;
+    loc[0] = __builtin_amdgcn_readfirstlane(int(unsigned(wave) / unsigned(waves)));
+    const int x = (wave - loc[0] * waves) * 64 + lane;
+    if (loc[0] >= bs0 || x >= n123) return;
+    // quotients of at most 511 by at most 64: half a step from an integer at least, far more
+    // than the reciprocal's error
+    loc[1] = int((float(x) + 0.5f) * __builtin_amdgcn_rcpf(float(n23)));
+    const int y = x - loc[1] * n23;
+    loc[2] = int((float(y) + 0.5f) * __builtin_amdgcn_rcpf(float(bs3)));
+    loc[3] = y - loc[2] * bs3;
+    p = loc[0] * n123 + x;
+  }
 
   // ---- children: per open dimension, AND the moves' children shifted along the child
   //      dimension (OR of complements = complement of AND), then apply the rest of the
@@ -251,20 +274,24 @@ __device__ __forceinline__ void fused_block(const BlockDev& B, const SecDev& S, 
   // ---- wins0, wins1 and the wins of every move (pentago/base/superscore.cc:38-96 pattern
   //      groups), one 64-bit word at a time: every reduction except the one over r3 stays
   //      inside a word, and the three groups reduced over r3 become ORs across words ----
-  NodeFields F;
+  NodeFields<kU> F;
 #pragma unroll
-  for (int a = 0; a < 2; a++)
+  for (int a = 0; a < kU; a++)
     F.glob[a] = fields + 4 * int64_t(S.field_off[a]) + 60 * int64_t(8 * bb[a] + loc[a]);
-  F.lds[0] = sf[0][loc[2]];
-  F.lds[1] = sf[1][loc[3]];
+#pragma unroll
+  for (int a = kU; a < 4; a++) F.lds[a - kU] = sf[a - kU][loc[a]];
   uint64_t A[3] = {0, 0, 0}, Bv[3] = {0, 0, 0}, Cv[3] = {0, 0, 0};
 #pragma unroll
   for (int k = 0; k < 4; k++) {
     uint64_t x[3];
     g2_acc(F, k, 0, FH, 2, FH, A);
     PE_FENCE();
-    g2(F, k, 0, FV, 1, FV, x);   // both quadrants wave-uniform: scalar
-    for (int t = 0; t < 3; t++) Bv[t] |= x[t];
+    if (kU == 2) {   // both quadrants wave-uniform: scalar
+      g2(F, k, 0, FV, 1, FV, x);
+      for (int t = 0; t < 3; t++) Bv[t] |= x[t];
+    } else {
+      g2_acc(F, k, 0, FV, 1, FV, Bv);
+    }
     PE_FENCE();
     g3_term(F, k, 1, FLO, 0, FAS, 2, FLO, x);
     for (int t = 0; t < 3; t++) Cv[t] |= x[t];
@@ -324,7 +351,7 @@ __device__ __forceinline__ void fused_block(const BlockDev& B, const SecDev& S, 
   st(o + 4, o1);
 }
 
-template <bool S35>
+template <bool S35, int kU>
 __global__ __launch_bounds__(kThreads, kWaves)
 void fused_blocks_kernel(const BlockDev* __restrict__ blocks, const LineDev* __restrict__ lines,
                          const SecDev* __restrict__ secs, const uint64_t* __restrict__ fields,
@@ -341,7 +368,13 @@ void fused_blocks_kernel(const BlockDev* __restrict__ blocks, const LineDev* __r
   const int blk = int(blockIdx.x >> 3) / kParts * 8 + int(blockIdx.x & 7), part = int(blockIdx.x >> 3) % kParts;
   if (blk >= nblocks) return;
   const BlockDev& B = blocks[blk];
-  fused_block<S35>(B, secs[B.sec], lines, fields, movetab, refl, part);
+  const SecDev& S = secs[B.sec];
+  // workgroups past a partial block's waves have nothing to do
+  int n[4];
+#pragma unroll
+  for (int a = 0; a < 4; a++) n[a] = min(8, S.rmin_size[a] - 8 * B.b[a]);
+  if (part * (kThreads / 64) >= n[0] * (kU == 2 ? 8 : (n[1] * n[2] * n[3] + 63) >> 6)) return;
+  fused_block<S35, kU>(B, S, lines, fields, movetab, refl, part);
 }
 
 // The same blocks fed from device work queues to a persistent grid: heads[x] counts the
@@ -369,7 +402,7 @@ void fused_blocks_queue_kernel(const BlockDev* __restrict__ blocks, const LineDe
       continue;
     }
     const BlockDev& B = blocks[xcd * blocks_per_xcd + t / kParts];
-    fused_block<S35>(B, secs[B.sec], lines, fields, movetab, refl, t % kParts);
+    fused_block<S35, 2>(B, secs[B.sec], lines, fields, movetab, refl, t % kParts);
     __syncthreads();   // the block's staged fields are no longer read
   }
 }
@@ -401,7 +434,7 @@ void fused_line_kernel(const LineLaunch a, const uint64_t* __restrict__ fields,
   }
   B.accumulate = a.line.accumulate;
   B.out = a.line.output + 8 * int64_t(k) * a.line.block_stride;
-  fused_block<S35>(B, a.sec, &a.line, fields, movetab, refl, part);
+  fused_block<S35, 2>(B, a.sec, &a.line, fields, movetab, refl, part);
 }
 
 int64_t slab_index(const pe_slab& s, const int b[4]) {
@@ -482,12 +515,35 @@ static pe_status slab_lines(const pe_slab& out, int nch, const pe_slab* ch, std:
   return PE_OK;
 }
 
+// Ragged blocks, whose waves are at most four fifths as many with kU = 1, are launched apart, if
+// that saves the plan enough waves to pay for a second launch's start and end (about 60 us at 4 ns
+// a wave): 96 sections of slice 34 (103 M nodes in 155 M lanes) 15.1 -> 13.1 ms, 5^4 blocks of
+// slice 30 with 128 ragged ones 247 us in one launch, 267 in two.  Full blocks stay with kU = 2:
+// 10^4 blocks of slice 30 4.25 ms, 4.65 with kU = 1 (a fifth wave a SIMD fewer, for the third
+// quadrant's entries in the LDS).
+constexpr int64_t kRaggedWaves = 16384;
+static int part_ragged(std::vector<BlockDev>* blocks, const std::vector<SecDev>& secs) {
+  auto saved = [&](const BlockDev& B) {
+    const SecDev& S = secs[size_t(B.sec)];
+    int n[4];
+    for (int a = 0; a < 4; a++) n[a] = std::min(8, S.rmin_size[a] - 8 * B.b[a]);
+    const int w = (n[1] * n[2] * n[3] + 63) / 64;
+    return 5 * w <= 4 * n[1] ? n[0] * (n[1] - w) : 0;
+  };
+  int64_t all = 0;
+  for (const BlockDev& B : *blocks) all += saved(B);
+  if (all < kRaggedWaves) return int(blocks->size());
+  return int(std::stable_partition(blocks->begin(), blocks->end(), [&](const BlockDev& B) { return !saved(B); }) -
+             blocks->begin());
+}
+
 // Pack blocks, lines (with their child offsets and reflection symmetries), sections and
 // move tables into one device allocation (field tables come from the device's field pool).
-static pe_status pack_fused_plan(const std::vector<BlockDev>& blocks, const std::vector<LineHost>& lines,
+static pe_status pack_fused_plan(std::vector<BlockDev> blocks, const std::vector<LineHost>& lines,
                                  const std::vector<SecDev>& secs, const std::vector<uint16_t>& movetab,
                                  int64_t nodes, FusedPlan* plan, std::string* err) {
   if (blocks.size() > size_t(0x7fffffff) / kParts) { *err = "fused plan too large"; return PE_ERR_CAPACITY; }
+  plan->nfull = part_ragged(&blocks, secs);
   // blob: blocks | lines | sections | moves | offsets | symmetries
   std::vector<LineDev> devs(lines.size());
   std::vector<int64_t> offs;
@@ -782,7 +838,7 @@ pe_status fused_plan_create(int nout, const pe_slab* outs, int nch, const pe_sla
     secs.push_back(sec);
     std::vector<BlockDev>().swap(r.blocks);
   }
-  return pack_fused_plan(blocks, lines, secs, movetab, nodes, plan, err);
+  return pack_fused_plan(std::move(blocks), lines, secs, movetab, nodes, plan, err);
 }
 
 bool fused_line_eligible(const LineHost& h) {
@@ -858,7 +914,7 @@ pe_status fused_line_plan_create(const std::vector<LineHost>& jobs, FusedPlan* p
     }
     lines.push_back(std::move(h));
   }
-  return pack_fused_plan(blocks, lines, secs, movetab, nodes, plan, err);
+  return pack_fused_plan(std::move(blocks), lines, secs, movetab, nodes, plan, err);
 }
 
 pe_status fused_plan_run(const FusedPlan& plan, hipStream_t stream) {
@@ -891,12 +947,14 @@ pe_status fused_plan_run(const FusedPlan& plan, hipStream_t stream) {
   }
   // a dispatch counts at most 2^32 work-items (4096 per block): plans with more blocks run
   // as consecutive launches of at most kChunk blocks, each spread over the XCDs as above
-  for (int b0 = 0; b0 < plan.nblocks; b0 += kChunk) {
-    const int n = std::min(kChunk, plan.nblocks - b0);
+  for (int b0 = 0, n; b0 < plan.nblocks; b0 += n) {
+    const bool full = b0 < plan.nfull;
+    n = std::min(kChunk, (full ? plan.nfull : plan.nblocks) - b0);
     const int px = (n + 7) / 8;
-    hipLaunchKernelGGL(plan.s35 ? fused_blocks_kernel<true> : fused_blocks_kernel<false>,
-                       dim3(unsigned(int64_t(px) * kParts * 8)), dim3(kThreads), 0, stream, blocks + b0, lines, secs,
-                       T.fields, moves, refl, n);
+    const auto kernel = plan.s35 ? (full ? fused_blocks_kernel<true, 2> : fused_blocks_kernel<true, 1>)
+                                 : (full ? fused_blocks_kernel<false, 2> : fused_blocks_kernel<false, 1>);
+    hipLaunchKernelGGL(kernel, dim3(unsigned(int64_t(px) * kParts * 8)), dim3(kThreads), 0, stream, blocks + b0, lines,
+                       secs, T.fields, moves, refl, n);
     PE_HIP(hipGetLastError(), "fused_blocks_kernel launch");
   }
   return PE_OK;
