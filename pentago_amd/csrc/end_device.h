@@ -20,16 +20,20 @@ __device__ __forceinline__ void strides4(const int s[4], int st[4]) {
   st[3] = 1; st[2] = s[3]; st[1] = s[2] * s[3]; st[0] = s[1] * s[2] * s[3];
 }
 // One super (32 bytes) as two 16-byte loads / stores.
+// Nodes lie in device memory: loads and stores say so, since a pointer that came out of memory is a
+// flat one to the compiler, whose accesses wait for the LDS as well.
+typedef uint64_t Pair __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(1))) Pair GlobalPair;
 __device__ __forceinline__ S4 ld(const uint64_t* p) {
-  const ulonglong2* q = reinterpret_cast<const ulonglong2*>(p);
-  const ulonglong2 a = q[0], b = q[1];
+  const GlobalPair* q = reinterpret_cast<const GlobalPair*>(reinterpret_cast<uint64_t>(p));
+  const Pair a = q[0], b = q[1];
   S4 r; r.w[0] = a.x; r.w[1] = a.y; r.w[2] = b.x; r.w[3] = b.y;
   return r;
 }
 __device__ __forceinline__ void st(uint64_t* p, S4 v) {
-  ulonglong2* q = reinterpret_cast<ulonglong2*>(p);
-  q[0] = make_ulonglong2(v.w[0], v.w[1]);
-  q[1] = make_ulonglong2(v.w[2], v.w[3]);
+  GlobalPair* q = reinterpret_cast<GlobalPair*>(reinterpret_cast<uint64_t>(p));
+  q[0] = Pair{v.w[0], v.w[1]};
+  q[1] = Pair{v.w[2], v.w[3]};
 }
 
 }  // namespace pe

@@ -30,6 +30,7 @@
 #include <thread>
 #include <unordered_map>
 #include <tuple>
+#include <type_traits>
 #include <vector>
 
 #include "device.h"
@@ -111,14 +112,105 @@ __device__ __forceinline__ void g3_term(const NodeFields<kU>& F, int k, int a, i
 
 constexpr int kThreads = 256;
 constexpr int kParts = 4096 / kThreads;
+// Slots of a word in the nodes' LDS array, padded so that the four lanes of a quad, two words apart,
+// use different banks.
+constexpr int kRow = kThreads + 4;
 constexpr int kChunk = 1 << 19;   // blocks per grid launch: 2^31 work-items
 // Occupancy: each node's running OR over its dimensions (and then its output words) lives in
-// LDS (16 KB per workgroup, 24 KB with the field entries), so a wave needs 66 VGPRs and six
-// waves share a SIMD (the LDS limit); children are loaded one move at a time.  Measured on
-// the headline launch against keeping them in registers (123 VGPRs, four waves, moves loaded
-// three at a time): 157.4 vs 168.4 ms; two moves at a time 162.5.  The launch bound asks for
-// at least five waves' worth of registers.
-constexpr int kWaves = 5;
+// LDS (16 KB per workgroup, 24 KB with the field entries), so that six waves share a SIMD
+// (the LDS limit; 80 VGPRs at most).  14^4 + 6^4 blocks of slice 24: 17.7 ms, with five waves 18.8.
+constexpr int kWaves = 6;
+
+// A value of lane kPerm of each quad of lanes (quad_perm of four two-bit lane numbers).
+template <int kPerm>
+__device__ __forceinline__ uint32_t quad(uint32_t v) {
+  return uint32_t(__builtin_amdgcn_mov_dpp(int(v), kPerm, 0xf, 0xf, true));
+}
+template <int kPerm>
+__device__ __forceinline__ uint64_t quad64(uint64_t v) {
+  return uint64_t(quad<kPerm>(uint32_t(v))) | uint64_t(quad<kPerm>(uint32_t(v >> 32))) << 32;
+}
+constexpr int kFrom0 = 0x00, kFrom1 = 0x55, kFrom2 = 0xAA, kFrom3 = 0xFF;   // a lane of the quad to all
+constexpr int kXor1 = 0xB1, kXor2 = 0x4E;                                   // from lane j ^ 1, j ^ 2
+
+// A quarter of a node (two words) in each lane of a quad.
+struct Quarter { uint64_t w[2]; };
+
+// Four quarters a lane, q[i] the lane's quarter of the quad's node i, to the four quarters of its
+// own node: a transposition over the quad's lanes.
+template <int kPerm>
+__device__ __forceinline__ void quad_exchange(Quarter& a, Quarter& b, bool odd) {
+#pragma unroll
+  for (int w = 0; w < 2; w++) {
+    const uint64_t x = a.w[w], y = b.w[w];
+    const uint64_t xo = quad64<kPerm>(x), yo = quad64<kPerm>(y);
+    a.w[w] = odd ? yo : x;
+    b.w[w] = odd ? y : xo;
+  }
+}
+__device__ __forceinline__ void quad_transpose(Quarter q[4], int j) {
+  quad_exchange<kXor1>(q[0], q[1], (j & 1) != 0);
+  quad_exchange<kXor1>(q[2], q[3], (j & 1) != 0);
+  quad_exchange<kXor2>(q[0], q[2], (j & 2) != 0);
+  quad_exchange<kXor2>(q[1], q[3], (j & 2) != 0);
+}
+
+// A quarter from device memory (a pointer that came out of memory is a flat one to the compiler,
+// whose loads wait for the LDS as well).
+__device__ __forceinline__ Quarter ld_quarter(uint64_t address) {
+  typedef uint64_t u2 __attribute__((ext_vector_type(2)));
+  const u2 v = *reinterpret_cast<const __attribute__((address_space(1))) u2*>(address);
+  return Quarter{{v.x, v.y}};
+}
+
+__device__ __forceinline__ void st_quarter(uint64_t address, const Quarter& v) {
+  typedef uint64_t u2 __attribute__((ext_vector_type(2)));
+  __builtin_nontemporal_store(u2{v.w[0], v.w[1]}, reinterpret_cast<__attribute__((address_space(1))) u2*>(address));
+}
+// Orders the wave's LDS writes before its reads of other lanes' slots.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
+// acc &= q shifted along coordinate cd by the amount in `word`'s low two bits, the word of the lane
+// kPerm of the quad; `mask` is that lane's select mask for coordinate 0.  Shifts along coordinates 0-2 stay inside a
+// word.  One along 3 moves whole words: the load has moved them by two, the rest is the other
+// quarter of the super, in lane j ^ 1.
+template <int cd>
+__device__ __forceinline__ void quarter_and(Quarter& acc, const Quarter& q, uint32_t word, uint32_t mask) {
+  const uint32_t k = word & 3;
+  if (cd == 3) {
+    const uint64_t next = quad64<kXor1>(q.w[0]);
+    const uint32_t odd = 0u - (k & 1);
+    acc.w[0] &= select64(q.w[0], q.w[1], odd);
+    acc.w[1] &= select64(q.w[1], next, odd);
+  } else if (cd == 2) {
+    for (int i = 0; i < 2; i++) acc.w[i] &= q.w[i] >> (16 * k) | q.w[i] << ((64 - 16 * k) & 63);
+  } else if (cd == 1) {
+    typedef uint16_t h2 __attribute__((ext_vector_type(2)));
+    const uint16_t right = uint16_t(4 * k), left = uint16_t(16 - 4 * k) & 15;
+    for (int i = 0; i < 2; i++) {
+      uint32_t r[2];
+      for (int h = 0; h < 2; h++) {
+        const h2 x = __builtin_bit_cast(h2, uint32_t(q.w[i] >> (32 * h)));
+        r[h] = __builtin_bit_cast(uint32_t, x >> h2{right, right}) | __builtin_bit_cast(uint32_t, x << h2{left, left});
+      }
+      acc.w[i] &= uint64_t(r[0]) | uint64_t(r[1]) << 32;
+    }
+  } else {
+    const int left = 4 - k;
+    for (int i = 0; i < 2; i++) {
+      uint32_t r[2];
+      for (int h = 0; h < 2; h++) {
+        const uint32_t x = uint32_t(q.w[i] >> (32 * h));
+        r[h] = lop3_32<kSel>(x >> k, x << left, mask);
+      }
+      acc.w[i] &= uint64_t(r[0]) | uint64_t(r[1]) << 32;
+    }
+  }
+}
 
 // One output block of 4096 nodes, computed by 16 workgroups (`part` = which 256 nodes).
 // S35: blocks of 35-stone sections, whose one move fills the board (no child data).
@@ -159,16 +251,22 @@ __device__ __forceinline__ void fused_block(const BlockDev& B, const SecDev& S, 
     }
     __syncthreads();
   }
-  int loc[4], p;
+  // lanes past the block's nodes take part with a node of the block (the lanes of a quad load
+  // each other's children) and store nothing
+  int loc[4], p, p0 = 0, count = 64;   // kU = 1: the wave's first node and how many it has
+  bool valid;
   if (kU == 2) {
     loc[0] = wave >> 3, loc[1] = wave & 7, loc[2] = lane >> 3, loc[3] = lane & 7;
-    if (loc[0] >= bs0 || loc[1] >= bs1 || loc[2] >= bs2 || loc[3] >= bs3) return;
+    if (loc[0] >= bs0 || loc[1] >= bs1) return;
+    valid = loc[2] < bs2 && loc[3] < bs3;
+    loc[2] = min(loc[2], bs2 - 1), loc[3] = min(loc[3], bs3 - 1);
     p = ((loc[0] * bs1 + loc[1]) * bs2 + loc[2]) * bs3 + loc[3];
   } else {
     const int n23 = bs2 * bs3, n123 = bs1 * n23, waves = (n123 + 63) >> 6;
     loc[0] = __builtin_amdgcn_readfirstlane(int(unsigned(wave) / unsigned(waves)));
-    const int x = (wave - loc[0] * waves) * 64 + lane;
-    if (loc[0] >= bs0 || x >= n123) return;
+    if (loc[0] >= bs0) return;
+    const int x0 = (wave - loc[0] * waves) * 64 + lane, x = min(x0, n123 - 1);
+    valid = x == x0;
     // quotients of at most 511 by at most 64: half a step from an integer at least, far more
     // than the reciprocal's error
     loc[1] = int((float(x) + 0.5f) * __builtin_amdgcn_rcpf(float(n23)));
@@ -176,22 +274,43 @@ __device__ __forceinline__ void fused_block(const BlockDev& B, const SecDev& S, 
     loc[2] = int((float(y) + 0.5f) * __builtin_amdgcn_rcpf(float(bs3)));
     loc[3] = y - loc[2] * bs3;
     p = loc[0] * n123 + x;
+    p0 = loc[0] * n123 + (wave - loc[0] * waves) * 64;
+    count = n123 - (wave - loc[0] * waves) * 64;
   }
+
+  if (S35 && !valid) return;   // no children; and no branch around the stores for all that they need to sink into
 
   // ---- children: per open dimension, AND the moves' children shifted along the child
   //      dimension (OR of complements = complement of AND), then apply the rest of the
   //      local rotation and the rearrangement ----
   // the node's running OR over the dimensions, then its output, in LDS: its own 8 words
   // ([word][thread], so a wave's accesses are consecutive 8-byte slots), never shared
-  __shared__ uint64_t sacc[S35 ? 1 : 8][kThreads];
-  uint64_t* o = B.out + 8 * p;
+  __shared__ uint64_t sacc[S35 ? 1 : 8][kRow];
+  // The output slots move between the LDS and memory as the children do, a quad of lanes to a
+  // node: quarter lane & 3 of the wave's node 16 i + lane / 4.
+  auto slots = [&](int i, auto f) {
+    const int n = 16 * i + (lane >> 2), row0 = int(threadIdx.x & ~63u);
+    int q;
+    bool in;
+    if (kU == 2) {
+      q = ((loc[0] * bs1 + loc[1]) * bs2 + (n >> 3)) * bs3 + (n & 7);
+      in = (n >> 3) < bs2 && (n & 7) < bs3;
+    } else {
+      q = p0 + n;
+      in = n < count;
+    }
+    if (in) f(reinterpret_cast<uint64_t>(B.out) + 64 * uint64_t(uint32_t(q)) + 16 * (lane & 3), 2 * (lane & 3), row0 + n);
+  };
   if (!S35) {
     if (mode >= 3) {   // the partial left in the output slots by an earlier pass
-      const S4 a = ld(o), b = ld(o + 4);
-      for (int w = 0; w < 4; w++) {
-        sacc[w][threadIdx.x] = a.w[w];
-        sacc[4 + w][threadIdx.x] = b.w[w];
-      }
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        slots(i, [&](uint64_t at, int w, int t) {
+          const Quarter v = ld_quarter(at);
+          sacc[w][t] = v.w[0];
+          sacc[w + 1][t] = v.w[1];
+        });
+      wave_sync();
     } else {
       for (int w = 0; w < 8; w++) sacc[w][threadIdx.x] = 0;
     }
@@ -214,19 +333,52 @@ __device__ __forceinline__ void fused_block(const BlockDev& B, const SecDev& S, 
     const uint16_t* row = movetab + S.move_off[d] + 16 * (8 * bb[d] + loc[d]);
     const int nm = S.nmoves[d];
     const int last = L.child_length - 1;
-    const uint64_t* in = L.input + 8 * L.in_base;
-    S4 acc0, acc1;
-    for (int i = 0; i < 4; i++) acc0.w[i] = acc1.w[i] = ~uint64_t(0);
-    // one move at a time: its child's four loads, then its shift
+    // The four lanes of a quad read each of their four children together, 16 bytes a lane, and
+    // write their output so: with each lane at its own node's 64 bytes the L1 was the bound where
+    // the children are not (its data path 98 % busy on 14^4 + 6^4 blocks of slice 24: 19.7 ms, now
+    // 17.1, of which 0.6 by the stores; one line of 18^4 22.1 -> 20.7 us).  Shifts along
+    // coordinates 0-2 stay inside a word, those along 3 move whole words, so the moves are ANDed
+    // as quarters and each lane gets its own node's once per dimension.
+    const int j = lane & 3;
+    const uint64_t in = reinterpret_cast<uint64_t>(L.input + 8 * L.in_base) + (cd == 3 ? 32 * (j >> 1) : 16 * j);
+    const uint32_t flip = cd == 3 ? 16 * (j & 1) : 0;
+    Quarter acc[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) acc[i].w[0] = acc[i].w[1] = ~uint64_t(0);
+    // one move at a time: its children's loads, then their shifts
+    int e = row[0];
     for (int m = 0; m < nm; m++) {
-      const int e = row[m];
-      const int kk = e & 63;
-      const int64_t cidx = int64_t(kk) * L.in_kstride + (kk == last ? base_last : base) +
-                           int64_t(L.input_stride) * ((e >> 6) & 7);
-      const uint64_t* c = in + 8 * cidx;
-      const S4 c0 = ld(c), c1 = ld(c + 4);
-      acc0 = s4_and(acc0, shift_coord_var(c0, cd, e >> 9));
-      acc1 = s4_and(acc1, shift_coord_var(c1, cd, e >> 9));
+      const int kk = e & 63, k = e >> 9;
+      const int64_t cidx = int64_t(kk) * L.in_kstride + ((kk == last ? base_last : base) +
+                                                         __mul24(L.input_stride, (e >> 6) & 7));
+      // the child's offset, with the move's amount in its low bits
+      const uint64_t off = 64 * uint64_t(cidx);
+      const uint32_t hi = uint32_t(off >> 32), lo = uint32_t(off) | uint32_t(k) | (cd == 3 ? 16 * (k >> 1) : 0);
+      const uint32_t l0 = quad<kFrom0>(lo), l1 = quad<kFrom1>(lo), l2 = quad<kFrom2>(lo), l3 = quad<kFrom3>(lo);
+      auto load = [&](uint32_t l, uint32_t h) { return ld_quarter(in + (uint64_t(lop3_32<kAndXor>(l, flip, ~3u)) | uint64_t(h) << 32)); };
+      const Quarter q0 = load(l0, quad<kFrom0>(hi)), q1 = load(l1, quad<kFrom1>(hi)), q2 = load(l2, quad<kFrom2>(hi)),
+                    q3 = load(l3, quad<kFrom3>(hi));
+      const int next = row[m + 1];   // rows have 16 entries
+      auto all = [&](auto coordinate) {
+        constexpr int c = decltype(coordinate)::value;
+        const uint32_t mask = c == 0 ? 0x11111111u * (0xfu >> k) : 0;
+        quarter_and<c>(acc[0], q0, l0, c == 0 ? quad<kFrom0>(mask) : 0);
+        quarter_and<c>(acc[1], q1, l1, c == 0 ? quad<kFrom1>(mask) : 0);
+        quarter_and<c>(acc[2], q2, l2, c == 0 ? quad<kFrom2>(mask) : 0);
+        quarter_and<c>(acc[3], q3, l3, c == 0 ? quad<kFrom3>(mask) : 0);
+      };
+      e = next;
+      if (cd == 0) all(std::integral_constant<int, 0>());
+      else if (cd == 1) all(std::integral_constant<int, 1>());
+      else if (cd == 2) all(std::integral_constant<int, 2>());
+      else all(std::integral_constant<int, 3>());
+    }
+    quad_transpose(acc, j);
+    S4 acc0, acc1;
+#pragma unroll
+    for (int w = 0; w < 4; w++) {
+      acc0.w[w] = acc[w >> 1].w[w & 1];
+      acc1.w[w] = acc[2 + (w >> 1)].w[w & 1];
     }
     // child frame -> parent frame: X(commute[g][x] + y).  Unreflected lines use one of four
     // fixed symmetries (straight-line code); reflected ones have a per-node y.
@@ -252,13 +404,10 @@ __device__ __forceinline__ void fused_block(const BlockDev& B, const SecDev& S, 
     for (int w = 0; w < 4; w++) sacc[4 + w][threadIdx.x] |= x1.w[w];
   }
   if (partial_out) {   // rmax(A) | rmax(B) = rmax(A | B): the finishing pass applies it once
-    S4 a, b;
-    for (int w = 0; w < 4; w++) {
-      a.w[w] = sacc[w][threadIdx.x];
-      b.w[w] = sacc[4 + w][threadIdx.x];
-    }
-    st(o, a);
-    st(o + 4, b);
+    wave_sync();
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      slots(i, [&](uint64_t at, int w, int t) { st_quarter(at, Quarter{{sacc[w][t], sacc[w + 1][t]}}); });
     return;
   }
   if (!S35) {   // rmax in place: words 0-3 from the children's [0] halves, 4-7 from [1]
@@ -337,13 +486,23 @@ __device__ __forceinline__ void fused_block(const BlockDev& B, const SecDev& S, 
       o1.w[k] = (nl.w[k] & ~imm) | w0v.w[k];
     }
   }
-  if (!S35)
+  if (!S35) {   // words 0-3 are the child words' second half
+    wave_sync();
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      o0.w[k] = sacc[4 + k][threadIdx.x];
-      o1.w[k] = sacc[k][threadIdx.x];
-    }
-  if (mode == 1) {   // OR-merge with other dimensions' lines (block_store.cc:173-229)
+    for (int i = 0; i < 4; i++)
+      slots(i, [&](uint64_t at, int w, int t) {
+        Quarter v{{sacc[w ^ 4][t], sacc[(w ^ 4) + 1][t]}};
+        if (mode == 1) {   // OR-merge with other dimensions' lines (block_store.cc:173-229)
+          const Quarter u = ld_quarter(at);
+          v.w[0] |= u.w[0];
+          v.w[1] |= u.w[1];
+        }
+        st_quarter(at, v);
+      });
+    return;
+  }
+  uint64_t* o = B.out + 8 * p;
+  if (mode == 1) {
     o0 = s4_or(o0, ld(o));
     o1 = s4_or(o1, ld(o + 4));
   }
@@ -352,7 +511,7 @@ __device__ __forceinline__ void fused_block(const BlockDev& B, const SecDev& S, 
 }
 
 template <bool S35, int kU>
-__global__ __launch_bounds__(kThreads, kWaves)
+__global__ __launch_bounds__(kThreads, kU == 2 ? kWaves : kWaves - 1)   // kU = 1: five by the LDS
 void fused_blocks_kernel(const BlockDev* __restrict__ blocks, const LineDev* __restrict__ lines,
                          const SecDev* __restrict__ secs, const uint64_t* __restrict__ fields,
                          const uint16_t* __restrict__ movetab, const uint8_t* __restrict__ refl,
@@ -383,7 +542,7 @@ void fused_blocks_kernel(const BlockDev* __restrict__ blocks, const LineDev* __r
 // i % 8) and, once that is exhausted, from the other runs in turn; every pop past a run's
 // end fails, so each workgroup stops after at most eight failed pops.
 template <bool S35>
-__global__ __launch_bounds__(kThreads, kWaves)
+__global__ __launch_bounds__(kThreads, kWaves - 1)   // six would spill
 void fused_blocks_queue_kernel(const BlockDev* __restrict__ blocks, const LineDev* __restrict__ lines,
                                const SecDev* __restrict__ secs, const uint64_t* __restrict__ fields,
                                const uint16_t* __restrict__ movetab, const uint8_t* __restrict__ refl,
