@@ -37,11 +37,12 @@ static_assert(kTileClass <= kTileThreads, "a class is one round");
 // halves that those are made from), chain 1 the rest.  They are kept apart, each thread reads and
 // writes the slots of its own chain only.
 //
-// LDS of a tile: its entries as they are stored (classes of even l, then of odd l, of each chain 0,
-// then chain 1), and the wins of both players' stones on the low cells beside the tile's high
-// ones, halves of parity 0 and 1.
+// LDS of a tile (kAlone: of one chain of a tile): its entries as they are stored (classes of even l,
+// then of odd l, of each chain 0, then chain 1), and the wins of both players' stones on the low
+// cells beside the tile's high ones, halves of parity 0 and 1.
+template <bool kAlone>
 struct TileLds {
-  uint4 half[2 * kTileEntries];
+  uint4 half[(kAlone ? 1 : 2) * kTileEntries];
   uint4 wins[2][2][1 << kTileCells];
 };
 
@@ -106,9 +107,9 @@ __host__ __device__ __forceinline__ TileJob tile_job(const MidBoardDev& B, uint6
 }
 
 // Sweep one tile (`tile` counts from the board's first; negative: only take part in the
-// barriers) with the kTileThreads * kChains threads tid = 0.. of a workgroup: each thread both
-// chains, or with kChains = 2 the second kTileThreads threads the second chain.  Every tile of a
-// board runs the same number of barriers (low + 1).
+// barriers) with the threads tid = 0.. of a workgroup: kTileThreads that each take both chains
+// (kChains = 1), kTileThreads for each chain (2), or kTileThreads for the chain `alone` only (2 and
+// kAlone).  Every tile of a board runs the same number of barriers (low + 1).
 //
 // What bounds it: for a launch that fills the chip, the reads of the tiles one high stone up, 32
 // bytes a position and empty high cell; else the latency of one tile.  The half that a class
@@ -117,17 +118,18 @@ __host__ __device__ __forceinline__ TileJob tile_job(const MidBoardDev& B, uint6
 // every other; the sweep that follows, a barrier a class, touches the LDS only.  The loads of a
 // tile are two deep: its record, then the children's ranks of all its classes (two registers
 // each), the wins and the tiles above at once.  Ranks loaded a class ahead and first entries
-// looked up cell by cell took 9.5 against 7.5 us for a step of 26 stones; 26 stones 68 -> 58 us,
-// 18 stones 2.57 -> 2.48 ms, 65 boards of 18-30 stones 22.5 -> 19.0 ms in all.
-template <int kChains>
-__device__ __forceinline__ void mid_tile(const TileJob& J, int tile, TileLds& lds, int tid) {
+// looked up cell by cell took 9.5 against 7.5 us for a step of 26 stones.  One MI355X: 26 stones 68
+// -> 58 us, 18 stones 2.57 -> 2.29 ms, of which 0.19 by 8 waves a SIMD with a thread a chain, where
+// both chains a thread allow 5.
+template <int kChains, bool kAlone = false>
+__device__ __forceinline__ void mid_tile(const TileJob& J, int tile, TileLds<kAlone>& lds, int tid, int alone = 0) {
   // Loads of the tiles above in flight for a thread: slots of this tile times tiles (a chain's
-  // slots are two rounds of its threads, both chains' three).  Both chains 2 x 4 and 1 x 4 take
-  // 6 % and 14 % longer, 6 x 1 9 %.  One chain a thread serves launches that leave the chip idle:
-  // more tiles at once.
-  constexpr int kSlots = kChains == 2 ? 2 : 3, kAbove = kChains == 2 ? 5 : 2;
-  const int chain0 = kChains == 2 ? __builtin_amdgcn_readfirstlane(tid / kTileThreads) : 0;
-  const int t = kChains == 2 ? tid % kTileThreads : tid;   // member of a class
+  // slots are two rounds of its threads, both chains' three).  One chain a thread, in the 64
+  // registers of 8 waves a SIMD: 2 x 3 and 2 x 2 alike, 2 x 4 20 % longer (spills), 2 x 5 with 6 waves 17 %.
+  // Both: 2 x 4 and 1 x 4 take 6 % and 14 % longer, 6 x 1 9 %.
+  constexpr int kSlots = kChains == 2 ? 2 : 3, kAbove = kChains == 2 ? 3 : 2;
+  const int chain0 = kAlone ? alone : kChains == 2 ? __builtin_amdgcn_readfirstlane(tid / kTileThreads) : 0;
+  const int t = kChains == 2 && !kAlone ? tid % kTileThreads : tid;   // member of a class
   const int wave0 = __builtin_amdgcn_readfirstlane(t & ~63);
   const int lane = tid & 63;
   const int low = J.low, high = J.high, spots = low + high;
@@ -149,7 +151,7 @@ __device__ __forceinline__ void mid_tile(const TileJob& J, int tile, TileLds& ld
   for (int l = kTileCells; l >= 0; l--)
     if (wave0 < count(l)) kids[l] = row[l * kTileClass];
   if (tile >= 0)
-    for (int i = tid; i < 4 << low; i += kTileThreads * kChains) {   // player, mask, parity
+    for (int i = tid; i < 4 << low; i += kAlone ? kTileThreads : kTileThreads * kChains) {   // player, mask, parity
       const int player = i >> (low + 1), k = i & ((2 << low) - 1);
       const uint64_t first = player ? (uint64_t(1) << spots) + (uint64_t(q) << low) : uint64_t(p) << low;
       lds.wins[player][k & 1][k >> 1] = J.wins[2 * first + k];
@@ -190,7 +192,7 @@ __device__ __forceinline__ void mid_tile(const TileJob& J, int tile, TileLds& ld
           for (int u = 0; u < kSlots; u++) or4(acc[u], in[at[u]]);
         }
 #pragma unroll
-        for (int u = 0; u < kSlots; u++) lds.half[(e ? 2 * size[0] : 0) + at[u]] = acc[u];
+        for (int u = 0; u < kSlots; u++) lds.half[kAlone ? (e ? size[0] : 0) + at[u] - first : (e ? 2 * size[0] : 0) + at[u]] = acc[u];
       }
     }
   // first slots of the classes from the highest on, below the class's own chain 0
@@ -201,7 +203,7 @@ __device__ __forceinline__ void mid_tile(const TileJob& J, int tile, TileLds& ld
     if (l > low) continue;
     const int n = h + l, mover = n & 1, par = (n + J.ply) & 1, e = l & 1, c = count(l);
     at[e] -= c;
-    uint4* half = lds.half + (e ? 2 * size[0] : 0) + at[e];
+    uint4* half = lds.half + (e ? (kAlone ? 1 : 2) * size[0] : 0) + at[e];
     tile_barrier();   // the tiles above (first round) or class l + 1 are in the LDS
     if (wave0 < c) {
       const int r = min(t, c - 1);
@@ -215,10 +217,11 @@ __device__ __forceinline__ void mid_tile(const TileJob& J, int tile, TileLds& ld
         const int chain = chain0 + k;
         const bool notlose = (mover ^ chain) != 0;   // wave-uniform
         uint4 acc = make_uint4(0, 0, 0, 0);
-        if (nhigh) acc = half[chain * size[e] + r];
+        const int lc = kAlone ? 0 : chain;   // in the LDS
+        if (nhigh) acc = half[lc * size[e] + r];
         if (n == spots && notlose) acc = make_uint4(~0u, ~0u, ~0u, ~0u);   // the board is full: not lost
         auto kid = [&](int j) {
-          return kid_half[chain * size[e ^ 1] + int(kids[l].w[j >> 2] >> (8 * (j & 3)) & 0xff)];
+          return kid_half[lc * size[e ^ 1] + int(kids[l].w[j >> 2] >> (8 * (j & 3)) & 0xff)];
         };
 #pragma unroll
         for (int j = 0; j < kTileCells - l; j += 2) {
@@ -244,7 +247,7 @@ __device__ __forceinline__ void mid_tile(const TileJob& J, int tile, TileLds& ld
         }
         x = hrmax4(x, before);
         if (t < c) {
-          half[chain * size[e] + t] = x;
+          half[lc * size[e] + t] = x;
           if (own != kNotStored) {
             uint4* out = entry(own) + (chain * size[e] + at[e]);
             if (J.stream) store_stream(&out[t], x);

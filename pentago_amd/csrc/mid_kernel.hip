@@ -47,10 +47,6 @@ __global__ __launch_bounds__(256) void mid_prep_one_kernel(MidBoardDev B, int64_
 // tiles.  Runs of 1 / 4 / 16 / 64 tiles measured within 3 %, 16 the fastest; one run of an eighth
 // of the launch to each XCD is 20 % slower (the groups of a step differ in tile size).
 constexpr int kRun = 16;
-__device__ __forceinline__ int run_order() {
-  const int x = blockIdx.x & 7, y = blockIdx.x >> 3;
-  return (y / kRun * 8 + x) * kRun + y % kRun;
-}
 unsigned run_grid(int64_t tiles) { return unsigned((tiles + 8 * kRun - 1) / (8 * kRun) * (8 * kRun)); }
 // A step that writes more than this (24 KB a tile at most) than the L2s hold together, 32 MB, is
 // stored past them: 18 empty cells 2.51 -> 2.43 ms; a small step's reader finds it in the L2.
@@ -58,26 +54,30 @@ constexpr int kStreamTiles = 2048;
 
 // Step `step` of every board that has one: workgroup w sweeps tile w - prefix[b] of the
 // step's tiles of board b.
-__global__ __launch_bounds__(kTileThreads, 5) void mid_step_kernel(const MidBoardDev* __restrict__ boards,
-                                                                const int64_t* __restrict__ prefix, int nb,
-                                                                int step, int ntiles, MidTabsDev M) {
-  __shared__ TileLds lds;
-  const int w = run_order();
+__global__ __launch_bounds__(2 * kTileThreads, 8) void mid_step_kernel(const MidBoardDev* __restrict__ boards,
+                                                                     const int64_t* __restrict__ prefix, int nb,
+                                                                     int step, int ntiles, MidTabsDev M) {
+  __shared__ TileLds<false> lds;
+  const int x = blockIdx.x & 7, y = blockIdx.x >> 3;
+  const int w = (y / kRun * 8 + x) * kRun + y % kRun;
   if (w >= ntiles) return;
   const int b = find_board(prefix, nb, w);
   const int t = w - int(prefix[b]);
   const MidBoardDev& B = boards[b];
   const MidSched& S = M.sched[B.I.spots];
-  mid_tile<1>(tile_job(B, B.work, S, M, ntiles > kStreamTiles), S.first[step] + t, lds, int(threadIdx.x));
+  mid_tile<2>(tile_job(B, B.work, S, M, ntiles > kStreamTiles), S.first[step] + t, lds, int(threadIdx.x));
 }
 
 // A step of one board, by value: `ntiles` tiles from `first` on.
-template <int kChains>
-__global__ __launch_bounds__(kTileThreads * kChains, kChains == 2 ? 4 : 5) void mid_step_one_kernel(TileJob J, int first,
-                                                                                                  int ntiles) {
-  __shared__ TileLds lds;
-  const int w = run_order();
-  if (w < ntiles) mid_tile<kChains>(J, first + w, lds, int(threadIdx.x));
+// A step of one board, by value: `ntiles` tiles from `first` on, a workgroup each, or with kAlone a
+// workgroup for each chain of a tile.
+template <bool kAlone>
+__global__ __launch_bounds__((kAlone ? 1 : 2) * kTileThreads, 8) void mid_step_one_kernel(TileJob J, int first,
+                                                                                        int ntiles) {
+  __shared__ TileLds<kAlone> lds;
+  const int x = blockIdx.x & 7, y = int(blockIdx.x >> 3) / (kAlone ? 2 : 1);
+  const int w = (y / kRun * 8 + x) * kRun + y % kRun;
+  if (w < ntiles) mid_tile<2, kAlone>(J, first + w, lds, int(threadIdx.x), int(blockIdx.x >> 3 & 1));
 }
 
 }  // namespace
@@ -109,11 +109,12 @@ void mid_carve(MidBoardDev* B, uint8_t* base) {
   B->results = reinterpret_cast<pe_halfsupers*>(base + t + mid_work_bytes(B->I));
 }
 
-// Up to this many tiles a step's time is a tile's latency more than the chip's rate (1280 tiles
-// of 32 KB LDS are in flight at once): a thread for each chain of a tile, twice the waves.  One
-// MI355X, never / up to 512 / up to 4096 tiles: 26 stones 71.8 / 61.4 / 61.3 us, 22 stones 175 /
-// 161 / 158, 19 stones 917 / 914 / 905.
-constexpr int64_t kTwoChains = 4096;
+
+// Up to the number of tiles whose chains the chip holds at once (8 workgroups of 20 KB LDS a compute unit),
+// a step's time is a tile's latency, which is shorter with a workgroup for each chain: 26 stones 62
+// -> 58 us, 22 stones 153 -> 145, 20 stones 343 -> 331.  A larger step would be no faster so, and its small
+// workgroups leave no room in the LDS for other streams' (65 boards of 18-30 stones 18.1 -> 20.6 ms).
+constexpr int64_t kAloneTiles = 1024;
 
 pe_status mid_launch_board(const MidBoardDev& B, const DevTables& T, hipStream_t stream) {
   const int64_t total = mid_prep_entries(B.I);
@@ -124,11 +125,12 @@ pe_status mid_launch_board(const MidBoardDev& B, const DevTables& T, hipStream_t
     const int64_t tiles = mid_step_tiles(B.I, k);
     if (tiles <= 0) continue;
     const TileJob J = tile_job(B, B.work, S, T.mid, tiles > kStreamTiles);
-    const dim3 grid(run_grid(tiles));
-    if (tiles <= kTwoChains)
-      hipLaunchKernelGGL(mid_step_one_kernel<2>, grid, dim3(2 * kTileThreads), 0, stream, J, S.first[k], int(tiles));
+    if (tiles <= kAloneTiles)
+      hipLaunchKernelGGL(mid_step_one_kernel<true>, dim3(2 * run_grid(tiles)), dim3(kTileThreads), 0, stream, J, S.first[k],
+                         int(tiles));
     else
-      hipLaunchKernelGGL(mid_step_one_kernel<1>, grid, dim3(kTileThreads), 0, stream, J, S.first[k], int(tiles));
+      hipLaunchKernelGGL(mid_step_one_kernel<false>, dim3(run_grid(tiles)), dim3(2 * kTileThreads), 0, stream, J, S.first[k],
+                         int(tiles));
     PE_HIP(hipGetLastError(), "mid_step_one_kernel launch");
   }
   return PE_OK;
@@ -205,7 +207,7 @@ pe_status mid_solve_levels(const std::vector<MidInfo>& infos, uint8_t* arena, st
     const int64_t total = p[nb];
     if (total <= 0) continue;
     if (total > 0x7fff0000) { set_error("too many tiles in one midsolve launch"); return PE_ERR_CAPACITY; }
-    hipLaunchKernelGGL(mid_step_kernel, dim3(run_grid(total)), dim3(kTileThreads), 0, stream, dboards,
+    hipLaunchKernelGGL(mid_step_kernel, dim3(run_grid(total)), dim3(2 * kTileThreads), 0, stream, dboards,
                        dprefix + size_t(nb + 1) * (t + 1), nb, t, int(total), T.mid);
     PE_HIP(hipGetLastError(), "mid_step_kernel launch");
   }

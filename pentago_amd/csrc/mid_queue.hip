@@ -25,7 +25,7 @@ __global__ __launch_bounds__(kThreads, 4) void mid_boards_kernel(const MidBoardD
                                                                  uint8_t* __restrict__ work_base, int64_t work_stride,
                                                                  unsigned int* __restrict__ head, MidTabsDev M) {
   constexpr int kSub = kThreads / kTileThreads;
-  __shared__ TileLds lds[kSub];
+  __shared__ TileLds<false> lds[kSub];
   __shared__ int s_b;
   const int sub = __builtin_amdgcn_readfirstlane(int(threadIdx.x) / kTileThreads);
   uint64_t* work = reinterpret_cast<uint64_t*>(work_base + int64_t(blockIdx.x) * work_stride);
