@@ -93,6 +93,7 @@ enum : int {
   kSel = 0xE4,      // c ? a : b
   kOrAnd = 0xF8,    // a | (b & c)
   kAndXor = 0x28,   // (a ^ b) & c
+  kOrThenAnd = 0xA8, // (a | b) & c
   kXor3 = 0x96,     // a ^ b ^ c
   kAndAnd = 0x80,   // a & b & c
 };
@@ -265,10 +266,14 @@ PE_HD S4 rmax(S4 a) {
 // Table: per (quadrant, state) five supers (horizontal, vertical, diagonal lo, hi, assist).
 // OR-reductions over one coordinate axis:
 // (each stage ORs in the partner bit at distance s: mask ? x >> s : x << s)
+// red0 by 32-bit halves: the OR of a nibble in its lowest bit, times 15.
+PE_HD uint32_t red0_half(uint32_t x) {
+  x |= x >> 1;
+  x = lop3_32<kOrThenAnd>(x, x >> 2, 0x11111111u);
+  return (x << 4) - x;
+}
 PE_HD uint64_t red0(uint64_t x) {
-  x |= lop3<kSel>(x >> 1, x << 1, 0x5555555555555555ull);
-  x |= lop3<kSel>(x >> 2, x << 2, 0x3333333333333333ull);
-  return x;
+  return uint64_t(red0_half(uint32_t(x))) | uint64_t(red0_half(uint32_t(x >> 32))) << 32;
 }
 PE_HD uint64_t red1(uint64_t x) {
   x |= lop3<kSel>(x >> 4, x << 4, 0x0F0F0F0F0F0F0F0Full);
