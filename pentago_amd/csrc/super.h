@@ -246,18 +246,20 @@ PE_HD S4 transform_super(int g, int y, S4 c) { return rearrange(shift_local(c, y
 // Per word: the +-1 rotations of r0 (inside nibbles) and r1 (nibbles inside 16-bit chunks) as
 // masked selects; those of r2 (16-bit chunks c0..c3) OR to (c1|c3, c0|c2) in both halves,
 // a 16-bit rotation of the OR of the halves; those of r3 are the neighbouring words.
+PE_HD uint32_t rmax_half(uint32_t x, uint32_t others) {   // r0, r1 of 32 bits, ORed with others
+  const uint32_t a = lop3_32<kSel>(x >> 1, x << 3, 0x77777777u), b = lop3_32<kSel>(x >> 3, x << 1, 0x11111111u);
+  const uint32_t c = lop3_32<kSel>(x >> 4, x << 12, 0x0FFF0FFFu), d = lop3_32<kSel>(x >> 12, x << 4, 0x000F000Fu);
+  return lop3_32<kOr3>(lop3_32<kOr3>(a, b, c), d, others);
+}
 PE_HD S4 rmax(S4 a) {
   S4 r;
   for (int i = 0; i < 4; i++) {
-    const uint64_t x = a.w[i];
-    const uint64_t s0 = lop3<kSel>(x >> 1, x << 3, 0x7777777777777777ull) |
-                        lop3<kSel>(x >> 3, x << 1, 0x1111111111111111ull);
-    const uint64_t s1 = lop3<kSel>(x >> 4, x << 12, 0x0FFF0FFF0FFF0FFFull) |
-                        lop3<kSel>(x >> 12, x << 4, 0x000F000F000F000Full);
+    const uint64_t x = a.w[i], p = a.w[(i + 1) & 3], q = a.w[(i + 3) & 3];
     const uint32_t h = uint32_t(x) | uint32_t(x >> 32);
     const uint32_t h2 = h >> 16 | h << 16;
-    const uint64_t s2 = uint64_t(h2) | uint64_t(h2) << 32;
-    r.w[i] = lop3<kOr3>(lop3<kOr3>(s0, s1, s2), a.w[(i + 1) & 3], a.w[(i + 3) & 3]);
+    const uint32_t lo = rmax_half(uint32_t(x), lop3_32<kOr3>(h2, uint32_t(p), uint32_t(q)));
+    const uint32_t hi = rmax_half(uint32_t(x >> 32), lop3_32<kOr3>(h2, uint32_t(p >> 32), uint32_t(q >> 32)));
+    r.w[i] = uint64_t(lo) | uint64_t(hi) << 32;
   }
   return r;
 }
@@ -275,15 +277,26 @@ PE_HD uint32_t red0_half(uint32_t x) {
 PE_HD uint64_t red0(uint64_t x) {
   return uint64_t(red0_half(uint32_t(x))) | uint64_t(red0_half(uint32_t(x >> 32))) << 32;
 }
+// red1: the OR of a 16-bit chunk's nibbles in its lowest nibble, times 0x1111 (24-bit factors).
+PE_HD uint32_t mul24(uint32_t a, uint32_t b) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return uint32_t(__mul24(int(a), int(b)));
+#else
+  return a * b;
+#endif
+}
+PE_HD uint32_t red1_half(uint32_t x) {
+  x |= x >> 8;
+  x = lop3_32<kOrThenAnd>(x, x >> 4, 0x000F000Fu);
+  return mul24(x, 0x1111u);
+}
 PE_HD uint64_t red1(uint64_t x) {
-  x |= lop3<kSel>(x >> 4, x << 4, 0x0F0F0F0F0F0F0F0Full);
-  x |= lop3<kSel>(x >> 8, x << 8, 0x00FF00FF00FF00FFull);
-  return x;
+  return uint64_t(red1_half(uint32_t(x))) | uint64_t(red1_half(uint32_t(x >> 32))) << 32;
 }
 PE_HD uint64_t red2(uint64_t x) {
-  x = lop3<kOr3>(x, x >> 16, x << 48);
-  const uint64_t h = (x | (x >> 32)) & 0xFFFFFFFFull;
-  return h | h << 32;
+  uint32_t h = uint32_t(x) | uint32_t(x >> 32);
+  h |= h >> 16 | h << 16;
+  return uint64_t(h) | uint64_t(h) << 32;
 }
 PE_HD S4 reduce0(S4 a) { for (int i = 0; i < 4; i++) a.w[i] = red0(a.w[i]); return a; }
 PE_HD S4 reduce1(S4 a) { for (int i = 0; i < 4; i++) a.w[i] = red1(a.w[i]); return a; }
