@@ -92,18 +92,54 @@ template <int kU>
 __device__ __forceinline__ void g3_term(const NodeFields<kU>& F, int k, int a, int fa, int b, int fb, int c, int fc,
                                         uint64_t x[3]) {
   const uint64_t a0 = F.w(a, k, 0, fa), b0 = F.w(b, k, 0, fb), c0 = F.w(c, k, 0, fc);
+  const uint64_t bc0 = b0 & c0;
+  x[0] = a0 & bc0;
+  x[1] = lop3<kAndAnd>(F.w(a, k, 1, fa), F.w(b, k, 1, fb), F.w(c, k, 1, fc));
+  const uint64_t inner = lop3<kOrAnd>(F.w(b, k, 2, fb) & c0, b0, F.w(c, k, 2, fc));
+  x[2] = lop3<kOrAnd>(F.w(a, k, 2, fa) & bc0, a0, inner);
+}
+// The same ORed into acc.
+template <int kU>
+__device__ __forceinline__ void g3_acc(const NodeFields<kU>& F, int k, int a, int fa, int b, int fb, int c, int fc,
+                                       uint64_t acc[3]) {
+  const uint64_t a0 = F.w(a, k, 0, fa), b0 = F.w(b, k, 0, fb), c0 = F.w(c, k, 0, fc);
   if (a < kU && b < kU) {
     const uint64_t ab0 = a0 & b0, ab2 = (F.w(a, k, 2, fa) & b0) | (a0 & F.w(b, k, 2, fb));
-    x[0] = ab0 & c0;
-    x[1] = (F.w(a, k, 1, fa) & F.w(b, k, 1, fb)) & F.w(c, k, 1, fc);
-    x[2] = lop3<kOrAnd>(ab2 & c0, ab0, F.w(c, k, 2, fc));
+    acc[0] = lop3<kOrAnd>(acc[0], ab0, c0);
+    acc[1] = lop3<kOrAnd>(acc[1], F.w(a, k, 1, fa) & F.w(b, k, 1, fb), F.w(c, k, 1, fc));
+    acc[2] = lop3<kOrAnd>(lop3<kOrAnd>(acc[2], ab2, c0), ab0, F.w(c, k, 2, fc));
   } else {
     const uint64_t bc0 = b0 & c0;
-    x[0] = a0 & bc0;
-    x[1] = lop3<kAndAnd>(F.w(a, k, 1, fa), F.w(b, k, 1, fb), F.w(c, k, 1, fc));
+    acc[0] = lop3<kOrAnd>(acc[0], a0, bc0);
+    acc[1] = lop3<kOrAnd>(acc[1], F.w(a, k, 1, fa), F.w(b, k, 1, fb) & F.w(c, k, 1, fc));
     const uint64_t inner = lop3<kOrAnd>(F.w(b, k, 2, fb) & c0, b0, F.w(c, k, 2, fc));
-    x[2] = lop3<kOrAnd>(F.w(a, k, 2, fa) & bc0, a0, inner);
+    acc[2] = lop3<kOrAnd>(lop3<kOrAnd>(acc[2], F.w(a, k, 2, fa), bc0), a0, inner);
   }
+}
+// Terms that are reduced over r2, which joins the halves of a word: the OR of a term's halves.
+__device__ __forceinline__ uint32_t or_halves(uint64_t x) { return uint32_t(x) | uint32_t(x >> 32); }
+__device__ __forceinline__ uint32_t and_halves(uint32_t acc, uint64_t x, uint64_t y) {   // acc | x & y
+  return lop3_32<kOrAnd>(lop3_32<kOrAnd>(acc, uint32_t(x), uint32_t(y)), uint32_t(x >> 32), uint32_t(y >> 32));
+}
+__device__ __forceinline__ uint32_t and_halves(uint64_t x, uint64_t y) {
+  return lop3_32<kOrAnd>(uint32_t(x) & uint32_t(y), uint32_t(x >> 32), uint32_t(y >> 32));
+}
+template <int kU>
+__device__ __forceinline__ void g2_halves(const NodeFields<kU>& F, int k, int a, int fa, int b, int fb, uint32_t x[3]) {
+  const uint64_t a0 = F.w(a, k, 0, fa), b0 = F.w(b, k, 0, fb);
+  x[0] = and_halves(a0, b0);
+  x[1] = and_halves(F.w(a, k, 1, fa), F.w(b, k, 1, fb));
+  x[2] = and_halves(and_halves(F.w(a, k, 2, fa), b0), a0, F.w(b, k, 2, fb));
+}
+template <int kU>
+__device__ __forceinline__ void g3_halves(const NodeFields<kU>& F, int k, int a, int fa, int b, int fb, int c, int fc,
+                                          uint32_t x[3]) {
+  const uint64_t a0 = F.w(a, k, 0, fa), b0 = F.w(b, k, 0, fb), c0 = F.w(c, k, 0, fc);
+  // a is wave-uniform, c is not: a and b together first, which is scalar work if b is uniform too
+  const uint64_t ab0 = a0 & b0, ab2 = lop3<kOrAnd>(F.w(a, k, 2, fa) & b0, a0, F.w(b, k, 2, fb));
+  x[0] = and_halves(ab0, c0);
+  x[1] = and_halves(F.w(a, k, 1, fa) & F.w(b, k, 1, fb), F.w(c, k, 1, fc));
+  x[2] = and_halves(and_halves(ab2, c0), ab0, F.w(c, k, 2, fc));
 }
 
 // Compiler-only memory fence: keeps the field loads of one word from being hoisted above
@@ -429,7 +465,8 @@ __device__ __forceinline__ void fused_block(const BlockDev& B, const SecDev& S, 
     F.glob[a] = fields + 4 * int64_t(S.field_off[a]) + 60 * int64_t(8 * bb[a] + loc[a]);
 #pragma unroll
   for (int a = kU; a < 4; a++) F.lds[a - kU] = sf[a - kU][loc[a]];
-  uint64_t A[3] = {0, 0, 0}, Bv[3] = {0, 0, 0}, Cv[3] = {0, 0, 0};
+  uint64_t A[3] = {0, 0, 0}, Cv[3] = {0, 0, 0};
+  uint32_t Bh[3] = {0, 0, 0};   // the halves' OR
 #pragma unroll
   for (int k = 0; k < 4; k++) {
     uint64_t x[3];
@@ -437,26 +474,31 @@ __device__ __forceinline__ void fused_block(const BlockDev& B, const SecDev& S, 
     PE_FENCE();
     if (kU == 2) {   // both quadrants wave-uniform: scalar
       g2(F, k, 0, FV, 1, FV, x);
-      for (int t = 0; t < 3; t++) Bv[t] |= x[t];
+      for (int t = 0; t < 3; t++) Bh[t] |= or_halves(x[t]);
     } else {
-      g2_acc(F, k, 0, FV, 1, FV, Bv);
+      uint32_t h[3];
+      g2_halves(F, k, 0, FV, 1, FV, h);
+      for (int t = 0; t < 3; t++) Bh[t] |= h[t];
     }
     PE_FENCE();
-    g3_term(F, k, 1, FLO, 0, FAS, 2, FLO, x);
-    for (int t = 0; t < 3; t++) Cv[t] |= x[t];
+    g3_acc(F, k, 1, FLO, 0, FAS, 2, FLO, Cv);
     PE_FENCE();
   }
   S4 o0, o1, wv, w0v, w1v;
 #pragma unroll
   for (int k = 0; k < 4; k++) {
     uint64_t w[3], x[3], y[3];
+    uint32_t p[3], q[3];
     g2_term(F, k, 2, FV, 3, FV, x);
     g3_term(F, k, 0, FLO, 2, FAS, 3, FLO, y);
-    for (int t = 0; t < 3; t++) w[t] = red1(lop3<kOr3>(A[t], red0(x[t]), y[t])) | Cv[t];
+    for (int t = 0; t < 3; t++) w[t] = red1(lop3<kOr3>(A[t], red0(x[t]), y[t]));
     PE_FENCE();
-    g2_term(F, k, 1, FH, 3, FH, x);
-    g3_term(F, k, 0, FHI, 1, FAS, 3, FHI, y);
-    for (int t = 0; t < 3; t++) w[t] |= red2(lop3<kOr3>(Bv[t], red0(x[t]), y[t]));
+    g2_halves(F, k, 1, FH, 3, FH, p);
+    g3_halves(F, k, 0, FHI, 1, FAS, 3, FHI, q);
+    for (int t = 0; t < 3; t++) {
+      const uint32_t h = red2_half(lop3_32<kOr3>(Bh[t], red0_half(p[t]), q[t]));
+      w[t] = lop3<kOr3>(w[t], Cv[t], uint64_t(h) | uint64_t(h) << 32);
+    }
     PE_FENCE();
     g3_term(F, k, 1, FHI, 3, FAS, 2, FHI, x);
     for (int t = 0; t < 3; t++) w[t] |= red0(x[t]);

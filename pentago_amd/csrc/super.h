@@ -277,25 +277,19 @@ PE_HD uint32_t red0_half(uint32_t x) {
 PE_HD uint64_t red0(uint64_t x) {
   return uint64_t(red0_half(uint32_t(x))) | uint64_t(red0_half(uint32_t(x >> 32))) << 32;
 }
-// red1: the OR of a 16-bit chunk's nibbles in its lowest nibble, times 0x1111 (24-bit factors).
-PE_HD uint32_t mul24(uint32_t a, uint32_t b) {
-#ifdef __HIP_DEVICE_COMPILE__
-  return uint32_t(__mul24(int(a), int(b)));
-#else
-  return a * b;
-#endif
-}
-PE_HD uint32_t red1_half(uint32_t x) {
-  x |= x >> 8;
-  x = lop3_32<kOrThenAnd>(x, x >> 4, 0x000F000Fu);
-  return mul24(x, 0x1111u);
-}
+// red1 of both halves at once: a byte for each 16-bit chunk, the OR of its four nibbles in both of the
+// byte's, then the byte twice.
 PE_HD uint64_t red1(uint64_t x) {
-  return uint64_t(red1_half(uint32_t(x))) | uint64_t(red1_half(uint32_t(x >> 32))) << 32;
+  const uint32_t lo = uint32_t(x), hi = uint32_t(x >> 32);
+  uint32_t r = pe_perm(hi, lo, 0x06040200u) | pe_perm(hi, lo, 0x07050301u);
+  r = lop3_32<kOrThenAnd>(r, r >> 4, 0x0F0F0F0Fu);
+  r |= r << 4;
+  return uint64_t(pe_perm(0, r, 0x01010000u)) | uint64_t(pe_perm(0, r, 0x03030202u)) << 32;
 }
+// red2 of a word by the OR of its halves; both halves of the result are the same.
+PE_HD uint32_t red2_half(uint32_t h) { return h | (h >> 16 | h << 16); }
 PE_HD uint64_t red2(uint64_t x) {
-  uint32_t h = uint32_t(x) | uint32_t(x >> 32);
-  h |= h >> 16 | h << 16;
+  const uint32_t h = red2_half(uint32_t(x) | uint32_t(x >> 32));
   return uint64_t(h) | uint64_t(h) << 32;
 }
 PE_HD S4 reduce0(S4 a) { for (int i = 0; i < 4; i++) a.w[i] = red0(a.w[i]); return a; }
