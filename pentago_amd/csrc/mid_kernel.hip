@@ -145,6 +145,19 @@ pe_status mid_launch_prep(const MidBoardDev* boards, const int64_t* prefix, int 
   return PE_OK;
 }
 
+// One board in device memory of at least mid_board_bytes, its 19 results stored to `results` (device
+// or mapped host memory).
+pe_status mid_solve_one(const MidInfo& info, uint8_t* arena, pe_halfsupers* results, hipStream_t stream) {
+  DevTables T;
+  std::string err;
+  if (device_tables(&T, &err) != PE_OK) { set_error(err); return PE_ERR_DEVICE; }
+  MidBoardDev B{};
+  B.I = info;
+  mid_carve(&B, arena);
+  B.results = results;
+  return mid_launch_board(B, T, stream);
+}
+
 // Level-synchronous solve of many boards whose scratch lives in `arena` (device memory of
 // at least the sum of mid_board_bytes).  Results land in each board's scratch; the caller
 // copies them out (offsets returned in result_offsets).
@@ -155,13 +168,6 @@ pe_status mid_solve_levels(const std::vector<MidInfo>& infos, uint8_t* arena, st
   if (device_tables(&T, &err) != PE_OK) { set_error(err); return PE_ERR_DEVICE; }
   const int nb = int(infos.size());
   if (!nb) return PE_OK;
-  if (nb == 1) {
-    MidBoardDev B{};
-    B.I = infos[0];
-    mid_carve(&B, arena);
-    result_offsets->assign(1, size_t(reinterpret_cast<uint8_t*>(B.results) - arena));
-    return mid_launch_board(B, T, stream);
-  }
   std::vector<MidBoardDev> boards(nb);
   result_offsets->resize(nb);
   size_t off = 0;
