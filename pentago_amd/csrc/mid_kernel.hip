@@ -33,7 +33,10 @@ __global__ __launch_bounds__(256) void mid_prep_kernel(const MidBoardDev* __rest
                                                        int64_t total, DevTables T) {
   const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (t >= total) return;
-  const int b = find_board(prefix, nb, t);
+  // the wave's first board by one search in scalar loads; a lane is a few boards past it at most
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) & ~63);
+  int b = find_board(prefix, nb, int64_t(blockIdx.x) * blockDim.x + wave);
+  while (b + 1 < nb && prefix[b + 1] <= t) b++;
   mid_wins_entry(boards[b], t - prefix[b], T);
 }
 
