@@ -260,11 +260,12 @@ pe_status launch_all(const MidPlan& plan, hipStream_t stream) {
   PE_HIP(hipEventRecord(plan.events[0], stream), "hipEventRecord(fork)");
   for (int s = 0; s < L.streams; s++)
     PE_HIP(hipStreamWaitEvent(plan.streams[size_t(s)], plan.events[0], 0), "hipStreamWaitEvent(fork)");
-  for (size_t k = 0; k < L.big.size(); k++) {
-    const pe_status st = mid_launch_board(plan.big[k], plan.tables, plan.streams[size_t(L.big_stream[k])]);
-    if (st != PE_OK) return st;
-  }
-  const pe_status st = launch_small(plan, stream);
+  // The small boards' one kernel first: a plan's stream may share its hardware queue with the run
+  // stream, and behind that stream's large boards it would start when they are done (65 boards of
+  // 18-30 stones 18.1 ms either way, with a shared queue 19.3 against 25.8).
+  pe_status st = launch_small(plan, stream);
+  for (size_t k = 0; k < L.big.size() && st == PE_OK; k++)
+    st = mid_launch_board(plan.big[k], plan.tables, plan.streams[size_t(L.big_stream[k])]);
   if (st != PE_OK) return st;
   for (int s = 0; s < L.streams; s++) {
     PE_HIP(hipEventRecord(plan.events[size_t(s) + 1], plan.streams[size_t(s)]), "hipEventRecord(join)");
