@@ -90,7 +90,7 @@ void build_field_pool(std::vector<uint64_t>* out) {
             for (int f = 0; f < 5; f++) {
               o[15 * k + f] = f0[4 * f + k];
               o[15 * k + 5 + f] = f1[4 * f + k];
-              o[15 * k + 10 + f] = fm[f][k];
+              o[15 * k + 10 + f] = fm[f][k] | f0[4 * f + k];
             }
         }
       }

@@ -130,7 +130,7 @@ pe_status fused_line_launch(const LineHost& h, const void* input, void* output, 
 // Field pool (one per device, built once): for quadrant q, player to move `turn` and
 // moves flag m, one entry of 60 words per rotation-minimal quadrant (all buckets, in
 // rmin_flat order): for each super word k, tables [F0 (mover's side), F1 (other side), Fm
-// (OR over the mover's moves in q; zero when m = 0)] x 5 fields (word k of each
+// (F0 and, with m = 1, the OR over the mover's moves in q)] x 5 fields (word k of each
 // superwin_info field, pentago/base/superscore.cc:38-96).  A section's field_off[q] is
 // field_pool_off(q, turn, m, counts[q]) in supers (4 words).
 int64_t field_pool_words();

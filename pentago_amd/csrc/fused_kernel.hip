@@ -15,7 +15,9 @@
 //     wins0, which ~imm removes anyway, so OR_m super_wins(side0 + m) & ~imm equals
 //     OR_G reduce_G(OR_{d in G} Fm_d,G & AND_{q in G, q != d} F0_q,G) & ~imm, with
 //     Fm = OR over the moves of the moved quadrant's field (AND distributes over OR).
-//     The device's field pool holds F0, F1 and Fm per (quadrant, rotation-minimal index).
+//     The device's field pool holds F0, F1 and Fm | F0 per (quadrant, rotation-minimal index): a
+//     move only adds patterns, and what F0 alone adds are wins of wins0 again.  With F0 inside
+//     Fm a group of three is (Fm_a & Fm_b & Fm_c) & majority(F0_a, F0_b, F0_c).
 //   * rmax(A) | rmax(B) = rmax(A | B) and T_m = R_g o shift_{y_m}: the children are shifted
 //     and ORed per dimension, rearranged once per dimension, and rmax runs once per node.
 #include <hip/hip_runtime.h>
@@ -87,16 +89,14 @@ __device__ __forceinline__ void g2_term(const NodeFields<kU>& F, int k, int a, i
   x[1] = F.w(a, k, 1, fa) & F.w(b, k, 1, fb);
   x[2] = lop3<kOrAnd>(F.w(a, k, 2, fa) & b0, a0, F.w(b, k, 2, fb));
 }
-// a2 b0 c0 | a0 b2 c0 | a0 b0 c2, products of two wave-uniform quadrants first
+// a2 b0 c0 | a0 b2 c0 | a0 b0 c2 = a2 b2 c2 & majority(a0, b0, c0), since each x0 is in its x2
 template <int kU>
 __device__ __forceinline__ void g3_term(const NodeFields<kU>& F, int k, int a, int fa, int b, int fb, int c, int fc,
                                         uint64_t x[3]) {
   const uint64_t a0 = F.w(a, k, 0, fa), b0 = F.w(b, k, 0, fb), c0 = F.w(c, k, 0, fc);
-  const uint64_t bc0 = b0 & c0;
-  x[0] = a0 & bc0;
+  x[0] = lop3<kAndAnd>(a0, b0, c0);
   x[1] = lop3<kAndAnd>(F.w(a, k, 1, fa), F.w(b, k, 1, fb), F.w(c, k, 1, fc));
-  const uint64_t inner = lop3<kOrAnd>(F.w(b, k, 2, fb) & c0, b0, F.w(c, k, 2, fc));
-  x[2] = lop3<kOrAnd>(F.w(a, k, 2, fa) & bc0, a0, inner);
+  x[2] = lop3<kAndAnd>(F.w(a, k, 2, fa), F.w(b, k, 2, fb), F.w(c, k, 2, fc)) & lop3<kMajority>(a0, b0, c0);
 }
 // The same ORed into acc.
 template <int kU>
@@ -109,11 +109,10 @@ __device__ __forceinline__ void g3_acc(const NodeFields<kU>& F, int k, int a, in
     acc[1] = lop3<kOrAnd>(acc[1], F.w(a, k, 1, fa) & F.w(b, k, 1, fb), F.w(c, k, 1, fc));
     acc[2] = lop3<kOrAnd>(lop3<kOrAnd>(acc[2], ab2, c0), ab0, F.w(c, k, 2, fc));
   } else {
-    const uint64_t bc0 = b0 & c0;
-    acc[0] = lop3<kOrAnd>(acc[0], a0, bc0);
+    acc[0] = lop3<kOrAnd>(acc[0], a0, b0 & c0);
     acc[1] = lop3<kOrAnd>(acc[1], F.w(a, k, 1, fa), F.w(b, k, 1, fb) & F.w(c, k, 1, fc));
-    const uint64_t inner = lop3<kOrAnd>(F.w(b, k, 2, fb) & c0, b0, F.w(c, k, 2, fc));
-    acc[2] = lop3<kOrAnd>(lop3<kOrAnd>(acc[2], F.w(a, k, 2, fa), bc0), a0, inner);
+    acc[2] = lop3<kOrAnd>(acc[2], lop3<kAndAnd>(F.w(a, k, 2, fa), F.w(b, k, 2, fb), F.w(c, k, 2, fc)),
+                          lop3<kMajority>(a0, b0, c0));
   }
 }
 // Terms that are reduced over r2, which joins the halves of a word: the OR of a term's halves.

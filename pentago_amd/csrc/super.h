@@ -96,6 +96,7 @@ enum : int {
   kOrThenAnd = 0xA8, // (a | b) & c
   kXor3 = 0x96,     // a ^ b ^ c
   kAndAnd = 0x80,   // a & b & c
+  kMajority = 0xE8, // two of a, b, c
 };
 
 // Byte gather from the 8-byte value (hi:lo): byte k of the result is byte sel_k of it
