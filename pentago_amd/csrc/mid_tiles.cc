@@ -55,7 +55,12 @@ struct Extents {
     return true;
   }
   void give(int64_t tile, const std::vector<uint32_t>& at, int64_t border) {
-    for (uint32_t x : at) free.emplace_back(int64_t(x), tile);
+    int64_t end = -1;   // of the run before: tiles taken from one extent follow each other
+    for (uint32_t x : at) {
+      if (int64_t(x) == end && end != border) free.back().second += tile;
+      else free.emplace_back(int64_t(x), tile);
+      end = int64_t(x) + tile;
+    }
     std::sort(free.begin(), free.end());
     std::vector<std::pair<int64_t, int64_t>> m;
     for (const auto& f : free) {
@@ -205,14 +210,17 @@ MidTabsHost build() {
         size_t i = 0;
         for (uint32_t p = 0; p < 1u << S.high; p++) {
           if (__builtin_popcount(p) != g.a) continue;
-          for (uint32_t q = 0; q < 1u << S.high; q++) {
-            if ((p & q) || __builtin_popcount(q) != g.b) continue;
+          const uint32_t rest = ((1u << S.high) - 1) & ~p;
+          uint32_t q = rest;   // the subsets of rest in ascending order, 0 first
+          do {
+            q = (q - rest) & rest;
+            if (__builtin_popcount(q) != g.b) continue;
             const uint32_t code = code3[p] + 2 * code3[q];
             for (int par = 0; par < 2; par++)
               if (!g.half[par].empty()) T.bases[2 * (size_t(S.bases) + code) + size_t(par)] = g.half[par][i];
             T.tiles.push_back(MidTile{p, q, code, 0});
             i++;
-          }
+          } while (q != rest);
         }
       }
     }
@@ -228,28 +236,35 @@ MidTabs MidTabsHost::view() const {
 }
 
 std::vector<uint32_t> mid_records(const MidTabs& M) {
-  std::vector<uint32_t> out;
+  size_t tiles = 0;
+  for (int spots = 0; spots <= kMidSpots; spots++) tiles += size_t(M.sched[spots].first[M.sched[spots].steps]);
+  std::vector<uint32_t> out(kRecWords * tiles);
+  uint32_t* r = out.data();
   for (int spots = 0; spots <= kMidSpots; spots++) {
     const MidSched& S = M.sched[spots];
-    for (int t = S.tiles; t < S.tiles + S.first[S.steps]; t++) {
-      const MidTile& X = M.tiles[t];
-      const int d = __builtin_popcount(X.p) - __builtin_popcount(X.q);
-      uint32_t r[kRecWords] = {};
-      r[0] = X.p | X.q << 16;
-      for (int par = 0; par < 2; par++) r[kRecOwn + par] = M.bases[2 * (size_t(S.bases) + X.code) + size_t(par)];
+    const uint32_t* bases = M.bases + 2 * size_t(S.bases);
+    uint32_t sizes[23] = {}, counts[23][2] = {};   // by d + 11
+    for (int d = -11; d <= 11; d++)
       for (int l = 0; l <= S.low; l++) {
         const uint32_t n = uint32_t(M.classes[mid_class_row(S.low, d, l)].count());
-        r[kRecSizes] += n << (l & 1 ? 16 : 0);
-        r[kRecCounts + l / 4] |= n << (8 * (l % 4));
+        sizes[d + 11] += n << (l & 1 ? 16 : 0);
+        counts[d + 11][l / 4] |= n << (8 * (l % 4));
       }
+    for (int t = S.tiles; t < S.tiles + S.first[S.steps]; t++, r += kRecWords) {
+      const MidTile& X = M.tiles[t];
+      const int d = __builtin_popcount(X.p) - __builtin_popcount(X.q) + 11;
+      r[0] = X.p | X.q << 16;
+      for (int par = 0; par < 2; par++) r[kRecOwn + par] = bases[2 * X.code + uint32_t(par)];
+      r[kRecSizes] = sizes[d];
+      r[kRecCounts] = counts[d][0];
+      r[kRecCounts + 1] = counts[d][1];
       uint32_t c3 = 1;
       for (int c = 0, j = 0; c < S.high; c++, c3 *= 3) {
         if ((X.p | X.q) >> c & 1) continue;
-        for (int m = 0; m < 2; m++)
-          r[kRecUp + m * kRecUp1 + j] = M.bases[2 * (size_t(S.bases) + X.code + (m + 1u) * c3) + (m ? 0 : 1)];
+        r[kRecUp + j] = bases[2 * (X.code + c3) + 1];
+        r[kRecUp + kRecUp1 + j] = bases[2 * (X.code + 2 * c3)];
         j++;
       }
-      out.insert(out.end(), r, r + kRecWords);
     }
   }
   return out;
