@@ -244,13 +244,15 @@ PE_HD S4 transform_super(int g, int y, S4 c) { return rearrange(shift_local(c, y
 
 // rmax(f)(a) = OR over the 8 single-quadrant rotations b of f(a+b)
 // (pentago/base/superscore.h:245-306).
-// Per word: the +-1 rotations of r0 (inside nibbles) and r1 (nibbles inside 16-bit chunks) as
-// masked selects; those of r2 (16-bit chunks c0..c3) OR to (c1|c3, c0|c2) in both halves,
+// Per word: the +-1 rotations of r0 (inside nibbles) and r1 (nibbles inside 16-bit chunks) by 32-bit
+// halves; those of r2 (16-bit chunks c0..c3) OR to (c1|c3, c0|c2) in both halves,
 // a 16-bit rotation of the OR of the halves; those of r3 are the neighbouring words.
 PE_HD uint32_t rmax_half(uint32_t x, uint32_t others) {   // r0, r1 of 32 bits, ORed with others
   const uint32_t a = lop3_32<kSel>(x >> 1, x << 3, 0x77777777u), b = lop3_32<kSel>(x >> 3, x << 1, 0x11111111u);
-  const uint32_t c = lop3_32<kSel>(x >> 4, x << 12, 0x0FFF0FFFu), d = lop3_32<kSel>(x >> 12, x << 4, 0x000F000Fu);
-  return lop3_32<kOr3>(lop3_32<kOr3>(a, b, c), d, others);
+  // nibbles: the OR of a nibble and the one two on (bytes of a chunk exchanged), then neighbours
+  const uint32_t y = x | pe_perm(0, x, 0x02030001u);
+  const uint32_t c = lop3_32<kSel>(y >> 4, y << 4, 0x0F0F0F0Fu);
+  return lop3_32<kOr3>(a, b, c) | others;
 }
 PE_HD S4 rmax(S4 a) {
   S4 r;
