@@ -98,6 +98,17 @@ void block_give(int device, void* p, size_t cap) {
   if (p) (void)hipFree(p);
 }
 
+hipError_t device_available(size_t* bytes) {
+  size_t total = 0;
+  int dev = 0;
+  hipError_t e = hipMemGetInfo(bytes, &total);
+  if (e == hipSuccess) e = hipGetDevice(&dev);
+  if (e != hipSuccess || dev < 0 || dev >= kMaxDevices) return e;
+  std::lock_guard<std::mutex> lock(g_kept_mu);
+  if (g_kept[dev].ptr) *bytes += g_kept[dev].cap;
+  return hipSuccess;
+}
+
 pe_status device_tables(DevTables* out, std::string* err) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) { *err = "no HIP device"; return PE_ERR_DEVICE; }
@@ -636,8 +647,8 @@ pe_status mid_resolve_config(const pe_mid_config* in, MidConfig* out) {
   pe_mid_config c{};
   if (in) c = *in;
   if (c.workspace_budget <= 0) {
-    size_t free_b = 0, total_b = 0;
-    PE_HIP(hipMemGetInfo(&free_b, &total_b), "hipMemGetInfo");
+    size_t free_b = 0;
+    PE_HIP(device_available(&free_b), "hipMemGetInfo");
     c.workspace_budget = std::min<int64_t>(int64_t(200e9), int64_t(0.6 * double(free_b)));
   }
   const TunedMid& t = g_tuned[dev];

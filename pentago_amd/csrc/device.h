@@ -44,6 +44,10 @@ hipError_t device_malloc(void** p, size_t bytes);
 constexpr size_t kKeptBytes = size_t(4) << 30;
 hipError_t block_take(size_t bytes, size_t limit, void** p, size_t* cap);
 void block_give(int device, void* p, size_t cap);
+// Memory that device_malloc can hand out on the current device: what is free, and the kept block,
+// which default budgets count as the free memory that it was before (without it each plan's budget
+// would depend on the plan closed before).
+hipError_t device_available(size_t* bytes);
 
 // Grow-only device allocation reused across synchronous calls (callers serialize use and
 // have no work pending on it when it grows).

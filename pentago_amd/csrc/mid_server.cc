@@ -348,8 +348,8 @@ pe_status mid_server_create(const pe_mid_server_config* c, MidServer** out) {
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, S->device);
   int64_t budget = c ? c->workspace_budget : 0;
   if (budget <= 0) {
-    size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return fail(PE_ERR_DEVICE, "hipMemGetInfo failed");
+    size_t free_b = 0;
+    if (device_available(&free_b) != hipSuccess) return fail(PE_ERR_DEVICE, "hipMemGetInfo failed");
     budget = std::min<int64_t>(int64_t(100e9), int64_t(0.4 * double(free_b)));
   }
   const int nstreams = c && c->streams > 0 ? c->streams : 4;

@@ -1,0 +1,37 @@
+"""Memory that a closed plan leaves to the next one, as its caller sees it: budgets that default to
+the free memory."""
+import pytest
+
+import pentago_amd as P
+from pentago_amd.workloads import seeded_boards
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def device():
+    P.init()
+
+
+def solve(boards, **kw):
+    """A plan's whole life; its info() and answers."""
+    plan = P.MidPlan(boards, **kw)
+    info = plan.info()
+    plan.run()
+    got = P.results_to_lists(boards, plan.results())
+    plan.close()
+    return info, got
+
+
+def test_default_budget_after_a_closed_plan():
+    """The kept block is memory that the next plan may have: its default budget is the same."""
+    solve(seeded_boards(4, 3, 28, 30))      # first use of the kernels, small block
+    boards = seeded_boards(100, 90, 22, 22)
+    first, expect = solve(boards)
+    kept = first["workspace_bytes"]
+    assert kept > 1 << 30
+    second, got = solve(boards)
+    assert got == expect
+    assert second["workgroups"] == first["workgroups"]
+    # 60 % of the free memory, which the kept block must not take part of away
+    assert second["workspace_budget"] > first["workspace_budget"] - 0.1 * kept
