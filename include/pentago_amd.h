@@ -29,6 +29,13 @@ typedef enum {
  * pentago/base/precompute.cc) and upload them to the current device.
  * Replaces the generated tables of pentago/base/gen/tables.h. */
 pe_status pe_init(void);
+/* The library keeps the device memory of one closed batched plan (pe_mid_plan_*) a device, at
+ * most 4 GiB, for the next plan: memory that the driver has to clear first costs about 27 ms a
+ * GB.  Default budgets count it as free, and every allocation of the library that would fail
+ * takes it back first; other allocators of the process do not see it.  Its size on the current
+ * device (0: none), and a call that gives it back to the device. */
+int64_t pe_kept_memory_bytes(void);
+pe_status pe_release_kept_memory(void);
 const char* pe_last_error(void);
 /* SHA-1 digest (40 hex chars + NUL) of a named table, hashed as the reference hashes it. */
 pe_status pe_table_digest(const char* name, char out[41]);

@@ -140,6 +140,8 @@ def lib():
         P, V = C.POINTER, C.c_void_p
         sig = {
             "pe_init": (C.c_int, []),
+            "pe_kept_memory_bytes": (C.c_int64, []),
+            "pe_release_kept_memory": (C.c_int, []),
             "pe_last_error": (C.c_char_p, []),
             "pe_table_digest": (C.c_int, [C.c_char_p, C.c_char_p]),
             "pe_section_shape": (C.c_int, [P(Section), P(C.c_int32)]),
@@ -647,6 +649,16 @@ class MidPlan:
             self.close()
         except Exception:
             pass
+
+
+def kept_memory_bytes():
+    """Device memory that the library keeps from a closed MidPlan on the current device."""
+    return int(lib().pe_kept_memory_bytes())
+
+
+def release_kept_memory():
+    """pe_release_kept_memory: give that memory back to the device."""
+    _check(lib().pe_release_kept_memory(), "pe_release_kept_memory")
 
 
 def mid_schedule_info(boards, workspace_budget, small_spots=14, workgroups=1024, threads=512, streams=2):

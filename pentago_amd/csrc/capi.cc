@@ -28,7 +28,7 @@ pe_status slab_line_passes(const pe_slab& out, int nch, const pe_slab* ch, std::
 pe_status launch_fill_seeded(void* d_nodes, int64_t nodes, uint64_t seed, int64_t first, hipStream_t stream);
 
 pe_status mid_solve_levels(const std::vector<MidInfo>& infos, uint8_t* arena, std::vector<size_t>* result_offsets,
-                           hipStream_t stream, DeviceBuffer* desc_cache);
+                           hipStream_t stream, DeviceBuffer& desc_cache);
 pe_status mid_solve_one(const MidInfo& info, uint8_t* arena, pe_halfsupers* results, hipStream_t stream);
 int mid_queue_blocks_per_cu();
 pe_status mid_solve_noalloc(const pe_high_board& board, pe_halfsupers* results, hipStream_t stream);
@@ -215,6 +215,21 @@ pe_status pe_init(void) {
   std::string err;
   const pe_status s = device_tables(&D, &err);
   if (s != PE_OK) return fail(s, err);
+  return PE_OK;
+  PE_GUARD_END
+}
+
+int64_t pe_kept_memory_bytes(void) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return 0;
+  std::lock_guard<std::mutex> lock(g_kept_mu);
+  return g_kept[dev].ptr ? int64_t(g_kept[dev].cap) : 0;
+}
+
+pe_status pe_release_kept_memory(void) {
+  PE_GUARD_BEGIN
+  const Kept k = kept_out([](const Kept&) { return true; });
+  if (k.ptr) PE_HIP(hipFree(k.ptr), "hipFree(kept memory)");
   return PE_OK;
   PE_GUARD_END
 }
@@ -981,7 +996,7 @@ pe_status pe_midsolve_batch(int n, const pe_high_board* boards, pe_halfsupers (*
     return PE_OK;
   }
   std::vector<size_t> offs;
-  pe_status st = mid_solve_levels(infos, static_cast<uint8_t*>(arena), &offs, s, &desc_cache[dev]);
+  pe_status st = mid_solve_levels(infos, static_cast<uint8_t*>(arena), &offs, s, desc_cache[dev]);
   if (st == PE_OK) {
     for (int b = 0; b < n; b++) {
       PE_HIP(hipMemcpyAsync(results[b], static_cast<uint8_t*>(arena) + offs[b], sizeof(pe_halfsupers) * 19,

@@ -165,7 +165,7 @@ pe_status mid_solve_one(const MidInfo& info, uint8_t* arena, pe_halfsupers* resu
 // at least the sum of mid_board_bytes).  Results land in each board's scratch; the caller
 // copies them out (offsets returned in result_offsets).
 pe_status mid_solve_levels(const std::vector<MidInfo>& infos, uint8_t* arena, std::vector<size_t>* result_offsets,
-                           hipStream_t stream, DeviceBuffer* desc_cache) {
+                           hipStream_t stream, DeviceBuffer& desc_cache) {
   DevTables T;
   std::string err;
   if (device_tables(&T, &err) != PE_OK) { set_error(err); return PE_ERR_DEVICE; }
@@ -194,13 +194,8 @@ pe_status mid_solve_levels(const std::vector<MidInfo>& infos, uint8_t* arena, st
   std::vector<uint8_t> blob(bytes);
   std::memcpy(blob.data(), boards.data(), desc_bytes);
   std::memcpy(blob.data() + desc_bytes, prefix.data(), sizeof(int64_t) * prefix.size());
-  void* d = nullptr;
-  if (desc_cache) {
-    PE_HIP(desc_cache->reserve(bytes), "hipMalloc(mid descriptors)");
-    d = desc_cache->ptr;
-  } else {
-    PE_HIP(hipMallocAsync(&d, bytes, stream), "hipMallocAsync(mid descriptors)");
-  }
+  PE_HIP(desc_cache.reserve(bytes), "hipMalloc(mid descriptors)");
+  void* const d = desc_cache.ptr;
   PE_HIP(hipMemcpyAsync(d, blob.data(), bytes, hipMemcpyHostToDevice, stream), "hipMemcpyAsync(mid descriptors)");
   const auto* dboards = static_cast<const MidBoardDev*>(d);
   const auto* dprefix = reinterpret_cast<const int64_t*>(static_cast<uint8_t*>(d) + desc_bytes);
@@ -220,7 +215,6 @@ pe_status mid_solve_levels(const std::vector<MidInfo>& infos, uint8_t* arena, st
                        dprefix + size_t(nb + 1) * (t + 1), nb, t, int(total), T.mid);
     PE_HIP(hipGetLastError(), "mid_step_kernel launch");
   }
-  if (!desc_cache) PE_HIP(hipFreeAsync(d, stream), "hipFreeAsync(mid descriptors)");
   return PE_OK;
 }
 

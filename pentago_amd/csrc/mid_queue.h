@@ -60,7 +60,6 @@ struct MidPlan {
   MidConfig cfg{};
   MidLayout layout;
   std::vector<MidInfo> infos;
-  hipStream_t alloc_stream = nullptr;  // stream-ordered allocation (serving) or null
   uint8_t* mem = nullptr;              // layout.bytes
   size_t mem_cap = 0;                  // block_take's size when the plan holds such a block, else 0
   hipEvent_t done = nullptr;           // the end of the last run, for such a block
@@ -79,22 +78,21 @@ struct MidPlan {
   int64_t launches = 0;                // kernel launches per run, at most
 };
 
-// alloc_stream null: synchronous hipMalloc/hipMemcpy; else stream-ordered on it.  With
+// upload_stream null: the descriptors go up by a synchronous hipMemcpy; else on that stream.  With
 // pinned host memory `upload` of at least the layout's o_res bytes (which must stay untouched
-// until alloc_stream has passed the plan's first run), the descriptor upload is queued
-// without waiting; otherwise the call waits for the upload.
+// until upload_stream has passed the plan's first run), the upload is queued without
+// waiting; otherwise the call waits for the upload.
 // With `memory` of at least the layout's bytes the plan lives there (nothing is allocated,
 // the caller keeps the memory until the plan is destroyed and its runs have finished).
 pe_status mid_plan_create(const std::vector<MidInfo>& infos, const MidConfig& cfg, MidPlan* plan,
-                          hipStream_t alloc_stream = nullptr, void* upload = nullptr, size_t upload_bytes = 0,
+                          hipStream_t upload_stream = nullptr, void* upload = nullptr, size_t upload_bytes = 0,
                           void* memory = nullptr, size_t memory_bytes = 0);
 pe_status mid_plan_run(MidPlan& plan, hipStream_t stream);
 // Queue the copy of all results to host memory on `stream`; after the stream has been
 // synchronized, mid_plan_zero_tail clears the entries past each board's spots.
 pe_status mid_plan_copy_results(const MidPlan& plan, pe_halfsupers (*out)[19], hipStream_t stream);
 void mid_plan_zero_tail(const MidPlan& plan, pe_halfsupers (*out)[19]);
-// Gives the plan's memory back (stream-ordered on alloc_stream when it was allocated that way,
-// else block_give).
+// Gives the plan's own memory back (block_give).
 void mid_plan_destroy(MidPlan* plan);
 int mid_board_blocks_per_cu(int threads);
 

@@ -132,7 +132,7 @@ const char* mid_layout(const std::vector<MidInfo>& infos, const MidConfig& cfg, 
 }
 
 pe_status mid_plan_create(const std::vector<MidInfo>& infos, const MidConfig& cfg, MidPlan* plan,
-                          hipStream_t alloc_stream, void* upload, size_t upload_bytes, void* memory,
+                          hipStream_t upload_stream, void* upload, size_t upload_bytes, void* memory,
                           size_t memory_bytes) {
   DevTables T;
   std::string err;
@@ -146,7 +146,6 @@ pe_status mid_plan_create(const std::vector<MidInfo>& infos, const MidConfig& cf
   plan->cfg = cfg;
   plan->infos = infos;
   plan->tables = T;
-  plan->alloc_stream = alloc_stream;
   PE_HIP(hipGetDevice(&plan->device), "hipGetDevice");
   int cus = 0;
   PE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, plan->device), "hipDeviceGetAttribute(CUs)");
@@ -154,7 +153,6 @@ pe_status mid_plan_create(const std::vector<MidInfo>& infos, const MidConfig& cf
   void* mem = nullptr;
   plan->owns_mem = !(memory && L.bytes <= memory_bytes);
   if (!plan->owns_mem) mem = memory;
-  else if (alloc_stream) PE_HIP(hipMallocAsync(&mem, L.bytes, alloc_stream), "hipMallocAsync(mid batch)");
   else PE_HIP(block_take(L.bytes, size_t(cfg.budget), &mem, &plan->mem_cap), "hipMalloc(mid batch)");
   plan->mem = static_cast<uint8_t*>(mem);
   uint8_t* base = plan->mem;
@@ -185,15 +183,15 @@ pe_status mid_plan_create(const std::vector<MidInfo>& infos, const MidConfig& cf
     B.work = reinterpret_cast<uint64_t*>(slot + mid_table_bytes(B.I));
     B.results = res + 19 * size_t(L.big[k]);
   }
-  if (alloc_stream && upload && blob.size() <= upload_bytes) {
+  if (upload_stream && upload && blob.size() <= upload_bytes) {
     // pinned staging owned by the caller: the copy is queued, nothing waits
     std::memcpy(upload, blob.data(), blob.size());
-    PE_HIP(hipMemcpyAsync(base, upload, blob.size(), hipMemcpyHostToDevice, alloc_stream),
+    PE_HIP(hipMemcpyAsync(base, upload, blob.size(), hipMemcpyHostToDevice, upload_stream),
            "hipMemcpyAsync(mid batch)");
-  } else if (alloc_stream) {
-    PE_HIP(hipMemcpyAsync(base, blob.data(), blob.size(), hipMemcpyHostToDevice, alloc_stream),
+  } else if (upload_stream) {
+    PE_HIP(hipMemcpyAsync(base, blob.data(), blob.size(), hipMemcpyHostToDevice, upload_stream),
            "hipMemcpyAsync(mid batch)");
-    PE_HIP(hipStreamSynchronize(alloc_stream), "mid batch upload");   // blob is a local
+    PE_HIP(hipStreamSynchronize(upload_stream), "mid batch upload");   // blob is a local
   } else {
     PE_HIP(hipMemcpy(base, blob.data(), blob.size(), hipMemcpyHostToDevice), "hipMemcpy(mid batch)");
   }
@@ -337,8 +335,7 @@ void mid_plan_destroy(MidPlan* plan) {
   }
   for (hipEvent_t e : plan->events) (void)hipEventDestroy(e);
   if (plan->mem && plan->owns_mem) {
-    if (plan->alloc_stream) (void)hipFreeAsync(plan->mem, plan->alloc_stream);
-    else if (!plan->done || plan->captured || hipEventSynchronize(plan->done) != hipSuccess) (void)hipFree(plan->mem);
+    if (!plan->done || plan->captured || hipEventSynchronize(plan->done) != hipSuccess) (void)hipFree(plan->mem);
     else block_give(plan->device, plan->mem, plan->mem_cap);
   }
   if (plan->done) (void)hipEventDestroy(plan->done);

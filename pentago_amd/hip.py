@@ -34,6 +34,7 @@ def hip():
             "hipStreamWaitEvent": [C.c_void_p, C.c_void_p, C.c_uint],
             "hipLaunchHostFunc": [C.c_void_p, C.c_void_p, C.c_void_p],
             "hipGetErrorString": [C.c_int],
+            "hipGetLastError": [],
         }
         for name, args in sig.items():
             f = getattr(L, name)
@@ -67,7 +68,13 @@ class Buffer:
     def __init__(self, nbytes):
         self.nbytes = int(nbytes)
         p = C.c_void_p()
-        check(hip().hipMalloc(C.byref(p), max(self.nbytes, 1)), "hipMalloc(%d)" % self.nbytes)
+        code = hip().hipMalloc(C.byref(p), max(self.nbytes, 1))
+        if code != 0:   # the library may keep a closed plan's memory
+            from . import release_kept_memory
+            hip().hipGetLastError()   # or the next launch would report it
+            release_kept_memory()
+            code = hip().hipMalloc(C.byref(p), max(self.nbytes, 1))
+        check(code, "hipMalloc(%d)" % self.nbytes)
         self.ptr = p.value
 
     def __del__(self):

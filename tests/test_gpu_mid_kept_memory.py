@@ -1,8 +1,9 @@
 """Memory that a closed plan leaves to the next one, as its caller sees it: budgets that default to
-the free memory."""
+the free memory, and a call that gives it back."""
 import pytest
 
 import pentago_amd as P
+from pentago_amd import hip
 from pentago_amd.workloads import seeded_boards
 
 pytestmark = pytest.mark.gpu
@@ -35,3 +36,18 @@ def test_default_budget_after_a_closed_plan():
     assert second["workgroups"] == first["workgroups"]
     # 60 % of the free memory, which the kept block must not take part of away
     assert second["workspace_budget"] > first["workspace_budget"] - 0.1 * kept
+
+
+def test_kept_memory_can_be_released():
+    boards = seeded_boards(100, 90, 22, 22)
+    solve(boards)
+    kept = P.kept_memory_bytes()
+    assert kept > 1 << 30
+    free = hip.mem_info()[0]
+    P.release_kept_memory()
+    assert P.kept_memory_bytes() == 0
+    # freed or not: the driver's own count moves by a few MB beside it
+    assert hip.mem_info()[0] - free > kept // 2
+    P.release_kept_memory()      # nothing kept: nothing to do
+    _, got = solve(boards[:3])
+    assert got == P.midsolve_batch(boards[:3], mode=0)
