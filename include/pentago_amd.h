@@ -366,7 +366,9 @@ typedef struct {
   int32_t pad;
 } pe_mid_config;
 typedef struct {
-  int64_t small_boards, large_boards, launches, workspace_bytes;
+  int64_t small_boards, large_boards, launches;
+  int64_t workspace_bytes;    /* device memory held: what the plan needs (pe_mid_schedule_info) and an eighth
+                                 to spare, or a kept block of less than twice that; within the budget */
   int32_t workgroups, streams;
 } pe_mid_plan_stats;
 typedef struct pe_mid_plan pe_mid_plan;

@@ -776,7 +776,7 @@ pe_status pe_mid_plan_info(const pe_mid_plan* plan, pe_mid_plan_stats* info, pe_
     info->small_boards = int64_t(P.layout.small.size());
     info->large_boards = int64_t(P.layout.big.size());
     info->launches = P.launches;
-    info->workspace_bytes = int64_t(P.layout.bytes);
+    info->workspace_bytes = int64_t(P.mem_cap ? P.mem_cap : P.layout.bytes);
     info->workgroups = P.layout.workgroups;
     info->streams = P.layout.streams;
   }

@@ -51,3 +51,18 @@ def test_kept_memory_can_be_released():
     P.release_kept_memory()      # nothing kept: nothing to do
     _, got = solve(boards[:3])
     assert got == P.midsolve_batch(boards[:3], mode=0)
+
+
+def test_a_plan_reports_the_memory_that_it_holds():
+    """A plan in the kept block of a larger one holds that block, unless its budget is smaller."""
+    P.release_kept_memory()
+    large, small = seeded_boards(100, 90, 22, 22), seeded_boards(70, 91, 22, 22)
+    need = P.mid_schedule_info(small, int(200e9), workgroups=512, threads=512, streams=2)[1]
+    held = solve(large)[0]["workspace_bytes"]
+    assert need < held < 2 * need and P.kept_memory_bytes() == held
+    info, got = solve(small)
+    assert info["workspace_bytes"] == held
+    assert got == P.midsolve_batch(small, mode=0)
+    info, got = solve(small, workspace_budget=need)
+    assert info["workspace_bytes"] == need
+    assert got == P.midsolve_batch(small, mode=0)
