@@ -32,8 +32,9 @@ pe_status pe_init(void);
 /* The library keeps the device memory of one closed batched plan (pe_mid_plan_*) a device, at
  * most 4 GiB, for the next plan: memory that the driver has to clear first costs about 27 ms a
  * GB.  Default budgets count it as free, and every allocation of the library that would fail
- * takes it back first; other allocators of the process do not see it.  Its size on the current
- * device (0: none), and a call that gives it back to the device. */
+ * takes it back first, as does a plan whose budget has no room for both.  Other allocators of the
+ * process do not see it.  Its size on the current device (0: none), and a call that gives it back
+ * to the device. */
 int64_t pe_kept_memory_bytes(void);
 pe_status pe_release_kept_memory(void);
 const char* pe_last_error(void);

@@ -47,7 +47,7 @@ std::atomic<int> g_end_form[kMaxDevices];
 void set_error(const std::string& e) { g_error = e; }
 
 namespace {
-struct Kept { void* ptr = nullptr; size_t cap = 0; };
+struct Kept { void* ptr = nullptr; size_t cap = 0; int passed = 0; };   // passed: plans since that it did not fit
 std::mutex g_kept_mu;
 Kept g_kept[kMaxDevices];
 
@@ -58,7 +58,7 @@ Kept kept_out(F fits) {
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices) return Kept();
   std::lock_guard<std::mutex> lock(g_kept_mu);
   const Kept k = g_kept[dev];
-  if (!k.ptr || !fits(k)) return Kept();
+  if (!k.ptr || !fits(g_kept[dev])) return Kept();
   g_kept[dev] = Kept();
   return k;
 }
@@ -75,13 +75,16 @@ hipError_t device_malloc(void** p, size_t bytes) {
 }
 
 hipError_t block_take(size_t bytes, size_t limit, void** p, size_t* cap) {
-  const Kept k = kept_out([&](const Kept& b) { return b.cap >= bytes && b.cap <= limit && b.cap / 2 < bytes; });
-  if (k.ptr) {
+  const size_t fresh = std::min(std::max(limit, bytes), bytes + bytes / 8);
+  const auto fits = [&](const Kept& b) { return b.cap >= bytes && b.cap <= limit && b.cap / 2 < bytes; };
+  const Kept k = kept_out([&](Kept& b) { return fits(b) || (++b.passed, b.cap + fresh > limit); });
+  if (k.ptr && fits(k)) {
     *p = k.ptr;
     *cap = k.cap;
     return hipSuccess;
   }
-  *cap = std::min(std::max(limit, bytes), bytes + bytes / 8);
+  if (k.ptr) (void)hipFree(k.ptr);
+  *cap = fresh;
   const hipError_t e = device_malloc(p, *cap);
   if (e == hipSuccess || *cap == bytes) return e;
   (void)hipGetLastError();
@@ -90,10 +93,14 @@ hipError_t block_take(size_t bytes, size_t limit, void** p, size_t* cap) {
 }
 
 void block_give(int device, void* p, size_t cap) {
-  if (cap <= kKeptBytes && device >= 0 && device < kMaxDevices) {   // the newer block stays
+  if (cap <= kKeptBytes && device >= 0 && device < kMaxDevices) {
     std::lock_guard<std::mutex> lock(g_kept_mu);
-    std::swap(g_kept[device].ptr, p);
-    g_kept[device].cap = cap;
+    Kept& k = g_kept[device];
+    if (!k.ptr || k.cap <= cap || k.passed >= 2) {
+      std::swap(k.ptr, p);
+      k.cap = cap;
+      k.passed = 0;
+    }
   }
   if (p) (void)hipFree(p);
 }

@@ -39,8 +39,11 @@ hipError_t device_malloc(void** p, size_t bytes);
 // kKeptBytes.  Freed VRAM is cleared before it is handed out again, which costs a process that
 // makes a plan a batch about 27 ms a GB once the device has no clean memory left.
 // take: a block for `bytes` (its size in *cap, at most `limit` and less than twice `bytes`), the
-// kept one of the current device or a new one with an eighth to spare.  give: back from its
-// owner, who has waited for all work that uses it.  Thread-safe: a block has one owner.
+// kept one of the current device or a new one with an eighth to spare, beside which the kept one
+// stays only if both are within `limit`.  give: back from its owner, who has waited for all work
+// that uses it.  The larger block is kept (large and small batches in turn: the large ones find
+// theirs, 27 ms a GB), but one that two plans in a row could not use makes room for a smaller.
+// Thread-safe: a block has one owner.
 constexpr size_t kKeptBytes = size_t(4) << 30;
 hipError_t block_take(size_t bytes, size_t limit, void** p, size_t* cap);
 void block_give(int device, void* p, size_t cap);

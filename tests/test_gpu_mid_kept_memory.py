@@ -66,3 +66,34 @@ def test_a_plan_reports_the_memory_that_it_holds():
     info, got = solve(small, workspace_budget=need)
     assert info["workspace_bytes"] == need
     assert got == P.midsolve_batch(small, mode=0)
+
+
+def test_a_plan_and_the_kept_block_within_the_budget():
+    P.release_kept_memory()
+    small = seeded_boards(40, 92, 22, 22)
+    need = P.mid_schedule_info(small, int(200e9), workgroups=512, threads=512, streams=2)[1]
+    solve(seeded_boards(100, 90, 22, 22))
+    kept = P.kept_memory_bytes()
+    assert kept > 2 * need
+    plan = P.MidPlan(small, workspace_budget=kept + 2 * need)    # room for both
+    assert P.kept_memory_bytes() == kept
+    plan.close()
+    assert P.kept_memory_bytes() == kept                         # the larger block stays
+    plan = P.MidPlan(small, workspace_budget=kept)               # room for the kept block or the plan
+    assert plan.info()["workspace_bytes"] <= kept and P.kept_memory_bytes() == 0
+    plan.run()
+    assert P.results_to_lists(small, plan.results()) == P.midsolve_batch(small, mode=0)
+    plan.close()
+
+
+def test_the_larger_block_is_kept_while_it_is_used():
+    P.release_kept_memory()
+    large, small = seeded_boards(100, 90, 22, 22), seeded_boards(40, 92, 22, 22)
+    held = solve(large)[0]["workspace_bytes"]
+    for _ in range(3):                                           # in turn
+        own = solve(small)[0]["workspace_bytes"]
+        assert own < held // 2 and P.kept_memory_bytes() == held
+        assert solve(large)[0]["workspace_bytes"] == held
+    solve(small)
+    solve(small)                                                 # no large plan any more
+    assert P.kept_memory_bytes() == own
