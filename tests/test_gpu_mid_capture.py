@@ -1,0 +1,39 @@
+"""Runs of a batched plan captured into a caller's graph: its replays, what becomes of the plan's
+memory, and the launches that a plan reports."""
+import numpy as np
+import pytest
+
+import pentago_amd as P
+from pentago_amd.workloads import seeded_board, seeded_boards
+from tests.graph_capture import Captured
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def device():
+    P.init()
+
+
+def boards_of(stones, seed=5):
+    rng = np.random.default_rng(seed)
+    return [seeded_board(rng, s) for s in stones]
+
+
+@pytest.mark.parametrize("streams", [-1, 2])
+def test_captured_run_and_closed_plan(streams):
+    """Replays equal eager runs; the memory of a plan that was captured is not handed on, since a
+    replay of the caller's may still use it."""
+    P.release_kept_memory()
+    boards = seeded_boards(40, 61, 20, 32)
+    expect = P.midsolve_batch(boards, mode=0)
+    plan = P.MidPlan(boards, streams=streams, use_graph=False)
+    graph = Captured(plan.run)
+    for _ in range(3):
+        graph.replay()
+        assert P.results_to_lists(boards, plan.results(graph.stream.ptr)) == expect
+        plan.run()
+        assert P.results_to_lists(boards, plan.results()) == expect
+    graph.close()
+    plan.close()
+    assert P.kept_memory_bytes() == 0
