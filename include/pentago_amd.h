@@ -359,8 +359,8 @@ typedef struct {
   int32_t small_spots;        /* boards with at most this many empty cells: one workgroup each (0: 14) */
   int32_t workgroups;         /* persistent workgroups for small boards (0: the tuned count when
                                  threads is the tuned size, else a full device of `threads`) */
-  int32_t threads;            /* threads per small-board workgroup: 256, 512, 1024 (0: 512); 512 becomes 1024 in
-                                 plans whose largest small boards are few */
+  int32_t threads;            /* threads per small-board workgroup: 256, 512, 1024 (0: 512, in plans whose
+                                 largest small boards are few 1024) */
   int32_t streams;            /* streams for large boards (0: 2; negative: all on the run stream) */
   int32_t use_graph;          /* > 0: pe_mid_plan_run replays a captured hipGraph; < 0: eager
                                  launches; 0: the device default (pe_mid_autotune's choice) */
@@ -386,11 +386,12 @@ pe_status pe_mid_plan_destroy(pe_mid_plan* plan);
 pe_status pe_mid_schedule_info(int n, const pe_high_board* boards, const pe_mid_config* config, int64_t* launches,
                                int64_t* workspace_bytes);
 /* Time candidate configurations on these boards (a warm-up, then the faster of two runs of the
- * whole batch each): the split small_spots in {12, 14, 16} at 512 threads, then 256 and 1024
- * threads at the best split, then the winner replayed as a captured hipGraph against eager
- * launches; the fastest becomes the current device's default.  Hand in the batch itself (or one like it): the best split
- * depends on how many boards of each size there are.  The chosen configuration is returned
- * through *best (use_graph 1 or -1). */
+ * whole batch each): the split small_spots in {12, 14, 16} with the threads that a plan with
+ * threads = 0 takes, then the other two of 256, 512 and 1024 threads at the best split, then the
+ * winner replayed as a captured hipGraph against eager launches.  The fastest becomes the current
+ * device's default (threads = 0 goes on choosing for each plan unless another size was faster).
+ * Hand in the batch itself (or one like it): the best split depends on how many boards of each
+ * size there are.  The chosen configuration is returned through *best (use_graph 1 or -1). */
 pe_status pe_mid_autotune(int n, const pe_high_board* boards, int64_t workspace_budget, pe_mid_config* best);
 
 /* Serving loop: single-position solve requests admitted as they arrive.  A worker thread

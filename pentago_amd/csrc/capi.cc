@@ -649,7 +649,7 @@ int64_t pe_midsolve_workspace_size(int min_slice) {
 
 namespace {
 
-struct TunedMid { bool set = false; int32_t small_spots = 0, threads = 0, workgroups = 0, use_graph = 0; };
+struct TunedMid { bool set = false; int32_t small_spots = 0, threads = 0, workgroups = 0, use_graph = 0; bool auto_threads = false; };
 TunedMid g_tuned[kMaxDevices];
 
 pe_status mid_infos(int n, const pe_high_board* boards, std::vector<MidInfo>* infos) {
@@ -675,6 +675,7 @@ pe_status mid_resolve_config(const pe_mid_config* in, MidConfig* out) {
   }
   const TunedMid& t = g_tuned[dev];
   if (c.small_spots <= 0) c.small_spots = t.set ? t.small_spots : 14;
+  out->auto_threads = c.threads <= 0 && (!t.set || t.auto_threads);
   if (c.threads <= 0) c.threads = t.set ? t.threads : 512;
   if (c.threads != 256 && c.threads != 512 && c.threads != 1024) return fail(PE_ERR_INVALID, "threads must be 256, 512 or 1024");
   // the tuned workgroup count belongs to the tuned workgroup size; another size given by the
@@ -744,6 +745,7 @@ pe_status pe_mid_schedule_info(int n, const pe_high_board* boards, const pe_mid_
   cfg.small_spots = config->small_spots;
   cfg.workgroups = config->workgroups;
   cfg.threads = config->threads;
+  cfg.auto_threads = false;
   cfg.streams = std::max(config->streams, 0);
   cfg.graph = false;
   MidLayout L;
@@ -792,7 +794,7 @@ pe_status pe_mid_plan_info(const pe_mid_plan* plan, pe_mid_plan_stats* info, pe_
     config->workspace_budget = P.cfg.budget;
     config->small_spots = P.cfg.small_spots;
     config->workgroups = P.cfg.workgroups;
-    config->threads = P.cfg.threads;
+    config->threads = P.board_threads;
     config->streams = P.cfg.streams;
     config->use_graph = P.cfg.graph;
   }
@@ -829,12 +831,14 @@ pe_status pe_mid_autotune(int n, const pe_high_board* boards, int64_t workspace_
   // handed in can be the real batch: the best split between the persistent small-board
   // kernel and the large boards' level launches depends on how many boards of each kind
   // there are
-  auto trial = [&](const pe_mid_config& c, float* ms) -> pe_status {
+  auto trial = [&](const pe_mid_config& c, bool auto_threads, float* ms, int* threads) -> pe_status {
     MidConfig cfg;
     pe_status r = mid_resolve_config(&c, &cfg);
     if (r != PE_OK) return r;
+    cfg.auto_threads = auto_threads;
     MidPlan plan;
     r = mid_plan_create(infos, cfg, &plan);
+    *threads = plan.board_threads;
     if (r == PE_OK) r = mid_plan_run(plan, s);   // untimed
     float best_t = -1;
     for (int rep = 0; rep < 2 && r == PE_OK; rep++) {
@@ -860,28 +864,36 @@ pe_status pe_mid_autotune(int n, const pe_high_board* boards, int64_t workspace_
     c.use_graph = graph;
     return c;
   };
-  // stage 1: the small/large split at 512 threads; stage 2: threads per small-board
-  // workgroup at that split; stage 3: the winner replayed as a captured graph
+  // stage 1: the small/large split with the threads chosen by the batch (board_threads); stage 2: the
+  // other sizes of a small-board workgroup at that split; stage 3: the winner replayed as a captured graph
   float best_ms = -1;
   pe_mid_config chosen{};
+  int threads = 0;            // of the winner, as run
+  bool auto_threads = true;   // the winner's were chosen by the batch: so are later plans'
   for (int32_t sm : {12, 14, 16}) {
     float ms = 0;
+    int th = 0;
     const pe_mid_config c = config(sm, 512, -1);
-    if ((st = trial(c, &ms)) != PE_OK) break;
-    if (best_ms < 0 || ms < best_ms) { best_ms = ms; chosen = c; }
+    if ((st = trial(c, true, &ms, &th)) != PE_OK) break;
+    if (best_ms < 0 || ms < best_ms) { best_ms = ms; chosen = c; threads = th; }
   }
-  if (st == PE_OK)
-    for (int32_t th : {256, 1024}) {
+  if (st == PE_OK) {
+    const int by_batch = threads;
+    for (int32_t th : {256, 512, 1024}) {
+      if (th == by_batch) continue;
       float ms = 0;
+      int as_run = 0;
       const pe_mid_config c = config(chosen.small_spots, th, -1);
-      if ((st = trial(c, &ms)) != PE_OK) break;
-      if (ms < best_ms) { best_ms = ms; chosen = c; }
+      if ((st = trial(c, false, &ms, &as_run)) != PE_OK) break;
+      if (ms < best_ms) { best_ms = ms; chosen = c; threads = th; auto_threads = false; }
     }
+  }
   if (st == PE_OK) {
     float ms = 0;
+    int th = 0;
     pe_mid_config c = chosen;
     c.use_graph = 1;
-    if ((st = trial(c, &ms)) == PE_OK && ms < best_ms) chosen.use_graph = 1;
+    if ((st = trial(c, auto_threads, &ms, &th)) == PE_OK && ms < best_ms) chosen.use_graph = 1;
   }
   if (st == PE_OK) {
     MidConfig cfg;
@@ -894,9 +906,11 @@ pe_status pe_mid_autotune(int n, const pe_high_board* boards, int64_t workspace_
   g_tuned[dev].set = true;
   g_tuned[dev].small_spots = chosen.small_spots;
   g_tuned[dev].threads = chosen.threads;
+  g_tuned[dev].auto_threads = auto_threads;
   g_tuned[dev].workgroups = chosen.workgroups;
   g_tuned[dev].use_graph = chosen.use_graph > 0;
   *best = chosen;
+  best->threads = threads;
   return PE_OK;
   PE_GUARD_END
 }

@@ -31,7 +31,8 @@ struct MidConfig {
   int64_t budget;        // bytes one run may hold (tables, workspaces, descriptors)
   int32_t small_spots;   // boards with at most this many empty cells: one workgroup each
   int32_t workgroups;    // persistent workgroups of the small-board kernel (upper bound)
-  int32_t threads;       // threads per small-board workgroup: 256, 512 (1024 where the largest boards are few) or 1024
+  int32_t threads;       // threads per small-board workgroup: 256, 512 or 1024
+  bool auto_threads;     // nobody asked for 512 threads: 1024 where the largest boards are few (board_threads)
   int32_t streams;       // streams carrying large boards (0: all work on the run stream)
   bool graph;            // replay the whole launch sequence through a captured hipGraph
 };
@@ -56,7 +57,7 @@ const char* mid_layout(const std::vector<MidInfo>& infos, const MidConfig& cfg, 
 struct MidPlan {
   int device = -1;
   int nb = 0;
-  int board_threads = 0;               // of a small board's workgroup (cfg.threads, or 1024 in place of 512)
+  int board_threads = 0;               // of a small board's workgroup (cfg.threads, or board_threads' 1024)
   MidConfig cfg{};
   MidLayout layout;
   std::vector<MidInfo> infos;

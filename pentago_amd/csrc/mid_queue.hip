@@ -50,17 +50,17 @@ __global__ __launch_bounds__(kThreads, 4) void mid_boards_kernel(const MidBoardD
 
 size_t up256(size_t x) { return (x + 255) & ~size_t(255); }
 
-// Threads of a small board's workgroup.  As many tiles are in flight on a compute unit with 1024 threads
+// Threads of a small board's workgroup where the caller leaves them open.  As many tiles are in flight on a compute unit with 1024 threads
 // as with 512, four of one board or two of each of two, so what differs is how long the largest boards
 // take: where a compute unit has at most one of them 1024 are better.  One MI355X, 512 / 1024: 64 boards of
 // 24-30 stones 1.34 / 0.99 ms, 1536 (219 of the largest) 2.03 / 1.61, 2048 (293) 2.17 / 2.39; 64 of 22-34
 // 11.8 / 8.5; boards of a single tile 512 up to 1024 boards 46 / 57 us.
-int board_threads(const std::vector<MidInfo>& infos, const MidLayout& L, int threads, int cus) {
-  if (threads != 512 || L.small.empty()) return threads;
+int board_threads(const std::vector<MidInfo>& infos, const MidLayout& L, const MidConfig& cfg, int cus) {
+  if (!cfg.auto_threads || L.small.empty()) return cfg.threads;
   const int top = infos[size_t(L.small[0])].spots;   // largest first
   int64_t n = 0;
   while (size_t(n) < L.small.size() && infos[size_t(L.small[size_t(n)])].spots == top) n++;
-  return top > kTileCells && n <= cus ? 1024 : threads;
+  return top > kTileCells && n <= cus ? 1024 : cfg.threads;
 }
 
 }  // namespace
@@ -149,7 +149,7 @@ pe_status mid_plan_create(const std::vector<MidInfo>& infos, const MidConfig& cf
   PE_HIP(hipGetDevice(&plan->device), "hipGetDevice");
   int cus = 0;
   PE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, plan->device), "hipDeviceGetAttribute(CUs)");
-  plan->board_threads = board_threads(infos, L, cfg.threads, cus);
+  plan->board_threads = board_threads(infos, L, cfg, cus);
   void* mem = nullptr;
   plan->owns_mem = !(memory && L.bytes <= memory_bytes);
   if (!plan->owns_mem) mem = memory;

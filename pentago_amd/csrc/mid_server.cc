@@ -358,6 +358,7 @@ pe_status mid_server_create(const pe_mid_server_config* c, MidServer** out) {
   S->cfg.budget = budget;
   S->cfg.small_spots = c && c->small_spots > 0 ? c->small_spots : 14;
   S->cfg.threads = 512;
+  S->cfg.auto_threads = true;
   S->cfg.workgroups = c && c->workgroups > 0 ? c->workgroups : cus * mid_board_blocks_per_cu(512) / nstreams;
   S->cfg.workgroups = std::max(S->cfg.workgroups, 1);
   S->cfg.streams = 0;   // a batch runs entirely on its server stream

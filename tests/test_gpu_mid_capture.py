@@ -37,3 +37,21 @@ def test_captured_run_and_closed_plan(streams):
     graph.close()
     plan.close()
     assert P.kept_memory_bytes() == 0
+
+
+@pytest.mark.parametrize("threads", [256, 512, 1024, 0])
+def test_threads_asked_for_are_run_and_reported(threads):
+    """Few boards of several tiles: the size that a plan without one asked for would change."""
+    boards = boards_of([26] * 3 + [30] * 4)
+    plan = P.MidPlan(boards, threads=threads, use_graph=False)
+    graph = Captured(plan.run)
+    info, blocks = plan.info(), sorted(b for _, b in graph.kernels())
+    graph.close()
+    assert info["large_boards"] == 0
+    assert blocks == sorted([1, 256, info["threads"]])     # queue head, tables, boards
+    if threads:
+        assert info["threads"] == threads
+    plan.run()
+    got = P.results_to_lists(boards, plan.results())
+    plan.close()
+    assert got == P.midsolve_batch(boards, mode=0)
