@@ -349,7 +349,7 @@ pe_status pe_midsolve_batch(int n, const pe_high_board* boards, pe_halfsupers (*
  * queue and solve each whole board (every step of tiles, workgroup barriers between steps) in
  * a workspace slot of their own; large boards step by step, one full-device launch per step
  * (at most one per level), on `streams` streams of their own that overlap with the small-board
- * kernel.  `launches` is an upper bound: a large board counts its tables and one per level.
+ * kernel.
  * Memory is held within workspace_budget (fewer workgroups / streams when it is tight).
  * No counterpart in the reference, which solves one board per call
  * (pentago/mid/midengine.cc:57-125); each board's results equal pe_midsolve_internal's.
@@ -381,7 +381,7 @@ pe_status pe_mid_plan_results(pe_mid_plan* plan, pe_halfsupers (*results)[19], v
 /* How the batch was split and the configuration in effect. */
 pe_status pe_mid_plan_info(const pe_mid_plan* plan, pe_mid_plan_stats* stats, pe_mid_config* config);
 pe_status pe_mid_plan_destroy(pe_mid_plan* plan);
-/* Host-only: the launches per run (an upper bound) and the device memory a plan with this (complete)
+/* Host-only: the most launches per run (a large board counts its tables and one a level) and the device memory a plan with this (complete)
  * configuration would use, or PE_ERR_CAPACITY.  No device calls. */
 pe_status pe_mid_schedule_info(int n, const pe_high_board* boards, const pe_mid_config* config, int64_t* launches,
                                int64_t* workspace_bytes);

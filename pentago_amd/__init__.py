@@ -662,7 +662,7 @@ def release_kept_memory():
 
 
 def mid_schedule_info(boards, workspace_budget, small_spots=14, workgroups=1024, threads=512, streams=2):
-    """pe_mid_schedule_info: (launches per run, device bytes) of a plan, host only."""
+    """pe_mid_schedule_info: (launches per run at most, device bytes) of a plan, host only."""
     n = len(boards)
     arr = (HighBoard * max(n, 1))(*boards)
     cfg = MidConfig(workspace_budget, small_spots, workgroups, threads, streams, 0, 0)

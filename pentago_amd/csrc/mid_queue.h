@@ -76,7 +76,7 @@ struct MidPlan {
   std::vector<hipStream_t> streams;    // owned, layout.streams of them
   std::vector<hipEvent_t> events;      // fork + one join per stream
   hipGraphExec_t graph_exec = nullptr;
-  int64_t launches = 0;                // kernel launches per run, at most
+  int64_t launches = 0;                // kernel launches per run
 };
 
 // upload_stream null: the descriptors go up by a synchronous hipMemcpy; else on that stream.  With

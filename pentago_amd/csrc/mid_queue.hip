@@ -211,7 +211,7 @@ pe_status mid_plan_create(const std::vector<MidInfo>& infos, const MidConfig& cf
     plan->events.push_back(ev);
   }
   int64_t launches = L.small.empty() ? 0 : 3;
-  for (int b : L.big) launches += 1 + infos[size_t(b)].spots + 1;
+  for (int b : L.big) launches += 1 + mid_steps(infos[size_t(b)]);
   plan->launches = launches;
   return PE_OK;
 }

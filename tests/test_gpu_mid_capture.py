@@ -55,3 +55,15 @@ def test_threads_asked_for_are_run_and_reported(threads):
     got = P.results_to_lists(boards, plan.results())
     plan.close()
     assert got == P.midsolve_batch(boards, mode=0)
+
+
+@pytest.mark.parametrize("stones", [[18], [19, 20, 21, 28, 29], [22, 35]])
+def test_launches_reported_are_launched(stones):
+    boards = boards_of(stones)
+    plan = P.MidPlan(boards, small_spots=8, use_graph=False)
+    graph = Captured(plan.run)
+    launched = len(graph.kernels())
+    graph.close()
+    assert plan.info()["launches"] == launched
+    assert P.mid_schedule_info(boards, int(200e9), small_spots=8)[0] >= launched
+    plan.close()
