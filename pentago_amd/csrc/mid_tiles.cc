@@ -236,12 +236,20 @@ MidTabs MidTabsHost::view() const {
 }
 
 std::vector<uint32_t> mid_records(const MidTabs& M) {
-  size_t tiles = 0;
-  for (int spots = 0; spots <= kMidSpots; spots++) tiles += size_t(M.sched[spots].first[M.sched[spots].steps]);
-  std::vector<uint32_t> out(kRecWords * tiles);
-  uint32_t* r = out.data();
+  int64_t tiles = 0;
+  for (int spots = 0; spots <= kMidSpots; spots++) tiles += M.sched[spots].first[M.sched[spots].steps];
+  std::vector<uint32_t> out(size_t(kRecWords * tiles));
+  mid_records(M, 0, tiles, out.data());
+  return out;
+}
+
+void mid_records(const MidTabs& M, int64_t first, int64_t n, uint32_t* r) {
+  std::fill(r, r + kRecWords * n, 0u);
   for (int spots = 0; spots <= kMidSpots; spots++) {
     const MidSched& S = M.sched[spots];
+    const int begin = int(std::max<int64_t>(S.tiles, first));
+    const int end = int(std::min<int64_t>(S.tiles + S.first[S.steps], first + n));
+    if (begin >= end) continue;
     const uint32_t* bases = M.bases + 2 * size_t(S.bases);
     uint32_t sizes[23] = {}, counts[23][2] = {};   // by d + 11
     for (int d = -11; d <= 11; d++)
@@ -250,7 +258,7 @@ std::vector<uint32_t> mid_records(const MidTabs& M) {
         sizes[d + 11] += n << (l & 1 ? 16 : 0);
         counts[d + 11][l / 4] |= n << (8 * (l % 4));
       }
-    for (int t = S.tiles; t < S.tiles + S.first[S.steps]; t++, r += kRecWords) {
+    for (int t = begin; t < end; t++, r += kRecWords) {
       const MidTile& X = M.tiles[t];
       const int d = __builtin_popcount(X.p) - __builtin_popcount(X.q) + 11;
       r[0] = X.p | X.q << 16;
@@ -267,7 +275,6 @@ std::vector<uint32_t> mid_records(const MidTabs& M) {
       }
     }
   }
-  return out;
 }
 
 std::vector<KidRanks> mid_kid_ranks(const MidTabs& M) {

@@ -96,6 +96,8 @@ struct MidTabsDev {
   const uint32_t* records;           // kRecWords a tile, in the order of MidTabs::tiles
   const KidRanks* kids;              // [mid_kid_row + rank]
 };
+// Records of n tiles from `first` on (kRecWords each); of all tiles.
+void mid_records(const MidTabs& M, int64_t first, int64_t n, uint32_t* out);
 std::vector<uint32_t> mid_records(const MidTabs& M);
 std::vector<KidRanks> mid_kid_ranks(const MidTabs& M);
 
