@@ -1,4 +1,6 @@
 // Tile records made in pieces against all of them at once.
+#include <stddef.h>
+
 #include <vector>
 
 #include "../../pentago_amd/csrc/mid_tiles.h"
