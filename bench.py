@@ -762,11 +762,12 @@ def mid_bench(P, hip, n_boards=4096, seed=2, tune=True, plain=True):
         plain_s = time.perf_counter() - t0
         log("midsolve plain: %.2f s" % plain_s)
         mism += int(np.sum(np.any(pres != res, axis=(1, 2))))
+    # each position's 32 bytes (both passes in one) written and read once
     work = 0
     from math import comb
     for sp in spots:
         sp = int(sp)
-        work += 2 * 16 * sum(comb(sp, n // 2) * comb(sp - n // 2, n - n // 2) * (sp - n + 1) for n in range(sp + 1))
+        work += 2 * 32 * sum(comb(sp, n // 2) * comb(sp - n // 2, n - n // 2) for n in range(sp + 1))
     if plain:
         # small boards alone (24..30 stones, 6..12 empty cells): launch overhead dominates the
         # plain path, the batched kernel solves them one workgroup per board
@@ -810,12 +811,11 @@ def mid_bench(P, hip, n_boards=4096, seed=2, tune=True, plain=True):
         "batched_over_plain": plain_s / batched_s if plain_s else None,
         "mismatches": mism, "plan": info,
         "algorithmic_GBps": work / batched_s / 1e9,
-        # HBM bound of the mix: its algorithmic bytes (32 B per position read or written, both
-        # passes in one) at 8 TB/s; batching cannot beat plain launches by more than
-        # plain time / this floor unless the kernels read less than the algorithmic bytes
+        # HBM bound of the mix: those bytes at 8 TB/s; batching cannot beat plain launches by
+        # more than plain time / this floor
         "roofline": {"bound": "hbm", "achieved": work / batched_s / 1e9, "peak": HBM_PEAK_GBPS, "unit": "GB/s",
                      "frac": work / batched_s / 1e9 / HBM_PEAK_GBPS, "traffic": mid_traffic(),
-                     "kernel": "batched plan (mid_step_kernel, mid_boards_kernel, mid_prep_kernel)",
+                     "kernel": "batched plan (mid_step_one_kernel, mid_boards_kernel, mid_prep kernels)",
                      "bytes_per_run": work, "run_ms": batched_s * 1e3},
         "hbm_floor_s": floor_s,
         "max_batched_over_plain_at_hbm_peak": plain_s / floor_s if plain_s else None,
