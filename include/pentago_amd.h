@@ -381,8 +381,9 @@ pe_status pe_mid_plan_results(pe_mid_plan* plan, pe_halfsupers (*results)[19], v
 /* How the batch was split and the configuration in effect. */
 pe_status pe_mid_plan_info(const pe_mid_plan* plan, pe_mid_plan_stats* stats, pe_mid_config* config);
 pe_status pe_mid_plan_destroy(pe_mid_plan* plan);
-/* Host-only: the most launches per run (a large board counts its tables and one a level) and the device memory a plan with this (complete)
- * configuration would use, or PE_ERR_CAPACITY.  No device calls. */
+/* Host-only: the most launches per run (a large board counts its tables and one a level) and the
+ * device memory that a plan with this (complete) configuration needs, or PE_ERR_CAPACITY.  No
+ * device calls. */
 pe_status pe_mid_schedule_info(int n, const pe_high_board* boards, const pe_mid_config* config, int64_t* launches,
                                int64_t* workspace_bytes);
 /* Time candidate configurations on these boards (a warm-up, then the faster of two runs of the

@@ -580,7 +580,7 @@ def midsolve_traverse(board, results):
 
 
 def midsolve_batch(boards, mode=0, stream=None):
-    """pe_midsolve_batch: mode 0 level-synchronous launches, 1 persistent work queue."""
+    """pe_midsolve_batch: mode 0 one launch a step over all boards, 1 persistent work queue."""
     n = len(boards)
     arr = (HighBoard * n)(*boards)
     res = ((HalfSupers * 19) * n)()
@@ -608,7 +608,7 @@ def results_to_lists(boards, res):
 
 class MidPlan:
     """A batch of boards solved by a batched plan (pe_mid_plan_*): small boards one per
-    workgroup through a persistent device-queue kernel, large boards level by level.
+    workgroup through a persistent device-queue kernel, large boards step by step.
 
     Build once, run any number of times; results() waits for the last run and returns an
     (n, 19, 4) uint64 array (win lo, win hi, notlose lo, notlose hi per entry)."""

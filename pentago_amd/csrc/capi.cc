@@ -879,7 +879,7 @@ pe_status pe_mid_autotune(int n, const pe_high_board* boards, int64_t workspace_
   // plan's first run touches freshly allocated workspace, and a graph candidate captures in
   // it; candidates differ by a few percent, about what one run varies by), so the boards
   // handed in can be the real batch: the best split between the persistent small-board
-  // kernel and the large boards' level launches depends on how many boards of each kind
+  // kernel and the large boards' step launches depends on how many boards of each kind
   // there are
   auto trial = [&](const pe_mid_config& c, bool auto_threads, float* ms, int* threads) -> pe_status {
     MidConfig cfg;

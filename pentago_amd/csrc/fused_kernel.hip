@@ -318,8 +318,9 @@ __device__ __forceinline__ void fused_block(const BlockDev& B, const SecDev& S, 
   // ---- children: per open dimension, AND the moves' children shifted along the child
   //      dimension (OR of complements = complement of AND), then apply the rest of the
   //      local rotation and the rearrangement ----
-  // the node's running OR over the dimensions, then its output, in LDS: its own 8 words
-  // ([word][thread], so a wave's accesses are consecutive 8-byte slots), never shared
+  // the node's running OR over the dimensions, then its output, in LDS: 8 words ([word][thread],
+  // so a wave's accesses are consecutive 8-byte slots) that its own thread works on; the wave's
+  // quads write them before (a partial) and read them after, across a wave_sync
   __shared__ uint64_t sacc[S35 ? 1 : 8][kRow];
   // The output slots move between the LDS and memory as the children do, a quad of lanes to a
   // node: quarter lane & 3 of the wave's node 16 i + lane / 4.

@@ -1,5 +1,4 @@
-// Midsolve device code shared by the level-synchronous and the work-queue kernels: the
-// per-board descriptor, the wins tables and the tile sweep (pentago/mid/internal.h:122-131 and
+// Midsolve device code shared by the step and the work-queue kernels: the wins tables and the tile sweep (pentago/mid/internal.h:122-131 and
 // 358-408, both aggressive passes at once; tiles: mid_tiles.h).
 #pragma once
 #include <hip/hip_runtime.h>
@@ -13,7 +12,8 @@
 namespace pe {
 
 // One entry of a board's wins tables: idx = player << spots | mask of empty cells, player 0 the
-// one to move at the root.  Masks with more stones than the player ever places are not read.
+// one to move at the root.  Masks with more stones than the player ever places are not written:
+// a tile copies them to its LDS with the rest and never uses them.
 __device__ inline void mid_wins_entry(const MidBoardDev& B, int64_t idx, const DevTables& T) {
   const int spots = B.I.spots;
   const int player = int(idx >> spots);

@@ -71,7 +71,6 @@ __global__ __launch_bounds__(2 * kTileThreads, 8) void mid_step_kernel(const Mid
   mid_tile<2>(tile_job(B, B.work, S, M, ntiles > kStreamTiles), S.first[step] + t, lds, int(threadIdx.x));
 }
 
-// A step of one board, by value: `ntiles` tiles from `first` on.
 // A step of one board, by value: `ntiles` tiles from `first` on, a workgroup each, or with kAlone a
 // workgroup for each chain of a tile.
 template <bool kAlone>
@@ -161,7 +160,7 @@ pe_status mid_solve_one(const MidInfo& info, uint8_t* arena, pe_halfsupers* resu
   return mid_launch_board(B, T, stream);
 }
 
-// Level-synchronous solve of many boards whose scratch lives in `arena` (device memory of
+// Solve of many boards, one launch a step over all of them, whose scratch lives in `arena` (device memory of
 // at least the sum of mid_board_bytes).  Results land in each board's scratch; the caller
 // copies them out (offsets returned in result_offsets).
 pe_status mid_solve_levels(const std::vector<MidInfo>& infos, uint8_t* arena, std::vector<size_t>* result_offsets,

@@ -10,7 +10,7 @@
 // the batch on that stream as a batched plan.  A board with more empty cells than the
 // small-board limit is a batch of its own and such batches hold at most all streams but
 // one, so the small boards' batches (one persistent kernel each, about a millisecond) are
-// never queued behind a large board's level launches.  Batches on different streams
+// never queued behind a large board's step launches.  Batches on different streams
 // overlap on the device.  Each request's state stays in device memory from admission to
 // retirement.
 #include <hip/hip_runtime.h>
@@ -135,7 +135,7 @@ struct MidServer {
       in_use -= b.bytes;
     }
     cv_done.notify_all();
-    mid_plan_destroy(&b.plan);   // stream-ordered free on the batch's stream
+    mid_plan_destroy(&b.plan);   // its memory is the stream's arena
     b = Batch();
     stream_busy[size_t(k)] = 0;
   }
@@ -243,9 +243,9 @@ struct MidServer {
         try {
           std::lock_guard<std::mutex> lock(mu);
           const auto now = Clock::now();
-          // A large board (more empty cells than small_spots: full-device level launches,
+          // A large board (more empty cells than small_spots: full-device step launches,
           // milliseconds) runs alone, on at most all streams but one; small boards batch
-          // together on the others, so they never wait behind a large board's levels.
+          // together on the others, so they never wait behind a large board's steps.
           int large_busy = 0;
           for (size_t j = 0; j < streams.size(); j++) large_busy += stream_busy[j] && batch_of_stream[j].large;
           const bool large_ok = streams.size() == 1 || large_busy + 1 < int(streams.size());

@@ -343,9 +343,7 @@ PE_HD S4 super_wins(uint64_t side, const uint64_t* table) {
 
 // ---------------- halfsupers (pentago/mid/halfsuper.h) ----------------
 // h(p)(a,b,c,d) = s(2a+(b+c+d+p)%2, b, c, d) at bit a + 2b + 8c + 32d.
-PE_HD H2 h2_not(H2 a) { a.w[0] = ~a.w[0]; a.w[1] = ~a.w[1]; return a; }
 PE_HD H2 h2_or(H2 a, H2 b) { a.w[0] |= b.w[0]; a.w[1] |= b.w[1]; return a; }
-PE_HD H2 h2_and(H2 a, H2 b) { a.w[0] &= b.w[0]; a.w[1] &= b.w[1]; return a; }
 
 PE_HD H2 split_half(S4 s, int parity) {
   H2 h; h.w[0] = h.w[1] = 0;

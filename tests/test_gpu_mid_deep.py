@@ -1,8 +1,8 @@
 """Midsolve at 18-21 stones (15-18 empty cells) on the GPU against the oracle, bit for bit.
 
-These are the boards whose levels run as full-device launches (mid_level_kernel on the plain
-path, mid_level1_kernel in batched plans, spread over the XCDs by s1p bands) or, up to the
-small-board limit, one workgroup each in the persistent queue kernel.  Every result entry
+These are the boards whose steps of tiles run as full-device launches (mid_step_one_kernel, on the
+plain path and in batched plans) or, up to the small-board limit, one workgroup each in the
+persistent queue kernel.  Every result entry
 (all 128 bits of win and notlose, root and children) is compared with the oracle's
 midsolve_internal (pentago/mid/midengine.cc:93-125), which the CPU suite pins bit for bit
 against brute-force search (pentago/mid/mid_test.cc:45-93 pattern).  The 163-value known

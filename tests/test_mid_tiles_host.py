@@ -1,6 +1,6 @@
 """The midsolve's tiles on the CPU (no GPU): where each tile is stored and read for every number
 of empty cells, and whole boards swept by the tables against the oracle, at the sizes around
-the tiles' eight low cells (one tile, the first high cells, several steps)."""
+the tiles' seven low cells (one tile, the first high cells, several steps)."""
 import ctypes as C
 import os
 import subprocess
