@@ -133,8 +133,8 @@ int64_t pe_end_plan_nodes(const pe_end_plan* plan);
 pe_status pe_end_plan_destroy(pe_end_plan* plan);
 /* Launch form of a plan's fused blocks (the blocks of every section of the plan, of any
  * size, in one launch).  0: a static grid, 16 workgroups per block.  n > 0: a persistent
- * grid of n workgroups per CU fed from device work queues, one per XCD over its share of the
- * blocks, workgroups taking from the other XCDs' queues once their own is empty.  The
+ * grid of n workgroups per CU fed from device work queues, one per XCD over that XCD's run
+ * of blocks, workgroups taking from the other XCDs' queues once their own is empty.  The
  * batched form of the reference's per-microline job pool (pentago/end/compute.cc:378-404).
  * Runs of one plan must not overlap (they share the queue heads). */
 pe_status pe_end_plan_set_launch(pe_end_plan* plan, int queue_wgs_per_cu);

@@ -579,23 +579,21 @@ void fused_blocks_kernel(const BlockDev* __restrict__ blocks, const LineDev* __r
 }
 
 // The same blocks fed from device work queues to a persistent grid: heads[x] counts the
-// tasks (16 parts a block) taken from XCD x's blocks, which are every eighth of the plan, as in
-// the grid.  A workgroup takes tasks of its own XCD (workgroup i runs on XCD i % 8) and, once
-// those are exhausted, of the others in turn; every pop past the end fails, so each workgroup
-// stops after at most eight failed pops.  Six workgroups a compute unit, a run of the plan to each
-// XCD / every eighth block: 14^4 + 6^4 blocks of slice 24 17.6 / 16.2 ms (shared children meet again),
-// the whole slice-30 section's dimension 0 136.9 / 133.2, its dimensions 1-3 128.9 / 130.8.
+// tasks (block * 16 + part, from the start of XCD x's run of blocks) taken from XCD x's
+// run.  A workgroup takes tasks from the run of its own XCD (workgroup i runs on XCD
+// i % 8) and, once that is exhausted, from the other runs in turn; every pop past a run's
+// end fails, so each workgroup stops after at most eight failed pops.
 template <bool S35>
 __global__ __launch_bounds__(kThreads, kWaves - 1)   // six would spill
 void fused_blocks_queue_kernel(const BlockDev* __restrict__ blocks, const LineDev* __restrict__ lines,
                                const SecDev* __restrict__ secs, const uint64_t* __restrict__ fields,
                                const uint16_t* __restrict__ movetab, const uint8_t* __restrict__ refl,
-                               int nblocks, unsigned int* __restrict__ heads) {
+                               int nblocks, int blocks_per_xcd, unsigned int* __restrict__ heads) {
   __shared__ int s_task;
   const int home = int(blockIdx.x) & 7;
   for (int x = 0; x < 8;) {
     const int xcd = (home + x) & 7;
-    const int run = (nblocks - xcd + 7) >> 3;
+    const int run = max(0, min(blocks_per_xcd, nblocks - xcd * blocks_per_xcd));
     if (threadIdx.x == 0) s_task = int(atomicAdd(&heads[xcd], 1u));
     __syncthreads();
     const int t = s_task;
@@ -604,7 +602,7 @@ void fused_blocks_queue_kernel(const BlockDev* __restrict__ blocks, const LineDe
       x++;
       continue;
     }
-    const BlockDev& B = blocks[t / kParts * 8 + xcd];
+    const BlockDev& B = blocks[xcd * blocks_per_xcd + t / kParts];
     fused_block<S35, 2>(B, secs[B.sec], lines, fields, movetab, refl, t % kParts);
     __syncthreads();   // the block's staged fields are no longer read
   }
@@ -1143,7 +1141,8 @@ pe_status fused_plan_run(const FusedPlan& plan, hipStream_t stream) {
     auto* heads = reinterpret_cast<unsigned int*>(base + plan.off_heads);
     hipLaunchKernelGGL(fused_queue_reset_kernel, dim3(1), dim3(64), 0, stream, heads);
     hipLaunchKernelGGL(plan.s35 ? fused_blocks_queue_kernel<true> : fused_blocks_queue_kernel<false>, dim3(grid),
-                       dim3(kThreads), 0, stream, blocks, lines, secs, T.fields, moves, refl, plan.nblocks, heads);
+                       dim3(kThreads), 0, stream, blocks, lines, secs, T.fields, moves, refl, plan.nblocks, per_xcd,
+                       heads);
     PE_HIP(hipGetLastError(), "fused_blocks_queue_kernel launch");
     return PE_OK;
   }
