@@ -31,7 +31,6 @@
 #include <string>
 #include <thread>
 #include <unordered_map>
-#include <tuple>
 #include <type_traits>
 #include <vector>
 
@@ -652,10 +651,10 @@ bool same_section(const pe_section& a, const pe_section& b) { return !std::memcm
 }  // namespace
 
 // Build the lines through an output slab (one per open dimension and cross-section block)
-// with child addressing into the child slabs.
+// with child addressing into the child slabs; dimension d's lines from first[d] on, in C order
+// over the box's other dimensions.
 static pe_status slab_lines(const pe_slab& out, int nch, const pe_slab* ch, std::vector<LineHost>* lines,
-                            std::map<std::tuple<int, int, int, int>, int>* index, std::string* err,
-                            uint32_t dims = 0xf) {
+                            size_t first[4], std::string* err, uint32_t dims = 0xf) {
   Section s;
   std::memcpy(s.c, out.section.counts, 8);
   int shape[4];
@@ -672,6 +671,7 @@ static pe_status slab_lines(const pe_slab& out, int nch, const pe_slab* ch, std:
   }
   for (int d = 0; d < 4; d++) {
     if (s.c[d][0] + s.c[d][1] >= 9 || !(dims >> d & 1)) continue;
+    first[d] = lines->size();
     int o[3], k = 0;
     for (int a = 0; a < 4; a++) if (a != d) o[k++] = a;
     for (int x = out.lo[o[0]]; x < out.hi[o[0]]; x++)
@@ -686,7 +686,6 @@ static pe_status slab_lines(const pe_slab& out, int nch, const pe_slab* ch, std:
           const pe_status st = make_line(L, &h, err);
           if (st != PE_OK) return st;
           if (h.dev.slice35) {   // the game ends after the move: no child data
-            (*index)[std::make_tuple(d, x, y, z)] = int(lines->size());
             lines->push_back(std::move(h));
             continue;
           }
@@ -709,7 +708,6 @@ static pe_status slab_lines(const pe_slab& out, int nch, const pe_slab* ch, std:
           int cb[4];
           for (int a = 0; a < 4; a++) cb[a] = h.info.first_child_block[a];
           for (int kk = 0; kk < h.info.input_blocks; kk++) { cb[cd] = kk; h.in_off.push_back(4096 * slab_index(*found, cb)); }
-          (*index)[std::make_tuple(d, x, y, z)] = int(lines->size());
           lines->push_back(std::move(h));
         }
   }
@@ -893,8 +891,8 @@ static void build_slab_body(const pe_slab& out, int nch, const pe_slab* ch, uint
                             SlabBuild* r) {
   const auto& Tb = tables();
   if (!out.data) { r->err = "output slab without memory"; r->status = PE_ERR_INVALID; return; }
-  std::map<std::tuple<int, int, int, int>, int> index;
-  r->status = slab_lines(out, nch, ch, &r->lines, &index, &r->err, dims);
+  size_t first_line[4] = {};
+  r->status = slab_lines(out, nch, ch, &r->lines, first_line, &r->err, dims);
   if (r->status != PE_OK) return;
   Section s;
   std::memcpy(s.c, out.section.counts, 8);
@@ -942,8 +940,7 @@ static void build_slab_body(const pe_slab& out, int nch, const pe_slab* ch, uint
   }
   std::vector<const LineHost*> first;
   for (int d = 0; d < 4; d++)
-    for (const LineHost& h : r->lines)
-      if (h.dev.dim == d) { first.push_back(&h); break; }
+    if (s.c[d][0] + s.c[d][1] < 9 && (dims >> d & 1)) first.push_back(&r->lines[first_line[d]]);
   order_by_symmetry(line_symmetries(first), lo, extent, &order);
   for (int64_t t : order) {
     int64_t rest = t;
@@ -959,9 +956,9 @@ static void build_slab_body(const pe_slab& out, int nch, const pe_slab* ch, uint
     for (int d = 0; d < 4; d++) {
       B.line[d] = -1;
       if (s.c[d][0] + s.c[d][1] >= 9 || !(dims >> d & 1)) continue;
-      int o[3], kk = 0;
-      for (int a = 0; a < 4; a++) if (a != d) o[kk++] = b[a];
-      B.line[d] = index.at(std::make_tuple(d, o[0], o[1], o[2]));
+      size_t cross = 0;
+      for (int a = 0; a < 4; a++) if (a != d) cross = cross * size_t(extent[a]) + size_t(b[a] - lo[a]);
+      B.line[d] = int(first_line[d] + cross);
     }
     B.out = static_cast<uint64_t*>(out.data) + 8 * 4096 * slab_index(out, b);
     r->blocks.push_back(B);
@@ -969,8 +966,8 @@ static void build_slab_body(const pe_slab& out, int nch, const pe_slab* ch, uint
   }
 }
 
-// Worker-thread entry: no exception leaves the thread (a host allocation failure or a bad
-// index becomes the slab's error status).
+// Worker-thread entry: no exception leaves the thread (a host allocation failure becomes the
+// slab's error status).
 static void build_slab(const pe_slab& out, int nch, const pe_slab* ch, uint32_t dims, int accumulate, SlabBuild* r) {
   try {
     build_slab_body(out, nch, ch, dims, accumulate, r);
@@ -1173,8 +1170,8 @@ void fused_plan_destroy(FusedPlan* plan) {
 pe_status slab_line_passes(const pe_slab& out, int nch, const pe_slab* ch, std::vector<std::vector<LineHost>>* passes,
                            int64_t* nodes_out, std::string* err) {
   std::vector<LineHost> lines;
-  std::map<std::tuple<int, int, int, int>, int> index;
-  pe_status st = slab_lines(out, nch, ch, &lines, &index, err);
+  size_t first_line[4] = {};
+  pe_status st = slab_lines(out, nch, ch, &lines, first_line, err);
   if (st != PE_OK) return st;
   Section s;
   std::memcpy(s.c, out.section.counts, 8);
