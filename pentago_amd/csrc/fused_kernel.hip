@@ -582,6 +582,10 @@ void fused_blocks_kernel(const BlockDev* __restrict__ blocks, const LineDev* __r
 // run.  A workgroup takes tasks from the run of its own XCD (workgroup i runs on XCD
 // i % 8) and, once that is exhausted, from the other runs in turn; every pop past a run's
 // end fails, so each workgroup stops after at most eight failed pops.
+// Every eighth block to an XCD, as in the grid, brings shared children together here too: 22^4 + 8^4
+// blocks of slice 24 105 -> 97 ms, level with the grid.  But ragged blocks have no form of their own here
+// (whole slice 35 11 ms, 5 in the grid), and a tuner that finds the two level would make this form the
+// default for them.
 template <bool S35>
 __global__ __launch_bounds__(kThreads, kWaves - 1)   // six would spill
 void fused_blocks_queue_kernel(const BlockDev* __restrict__ blocks, const LineDev* __restrict__ lines,
